@@ -1629,15 +1629,15 @@ int rtb_hall_energy_cut(const rtb_model* m, const size_t* kmesh, const double* m
   RTB_TRY(tmr.begin(RTB_STAGE_KUBO));
   RTB_TRY(energy_cut_omega(st, n, nk, dEv, dKv, dperm, eta, dom));
   RTB_TRY(tmr.end(1));
-  const size_t waves = energy_cut_waves(m->dim, nx, ny, nz, n);
-  const size_t chunk = std::max<size_t>(1, std::min<size_t>(256, (size_t(512) << 20) / (waves * sizeof(double))));
-  double* dpart;
-  RTB_TRY(w.alloc(&dpart, waves * chunk));
   const double width = T <= 0.0 ? 0.0 : T * 8.617333262145e-5;  // thermodynamics.rs:10, 50-59
   RTB_TRY(energy_cut_convolve(mu, n_mu, width, [&](const double* mv, size_t nm, double* s0) -> int {
-    double *dmu, *ds0;
+    // partial rows of at most 512 MB (at least one column)
+    const size_t rows = energy_cut_rows(m->dim, nx, ny, nz, n, nm);
+    const size_t chunk = std::max<size_t>(1, std::min<size_t>(nm, (size_t(512) << 20) / (rows * sizeof(double))));
+    double *dmu, *ds0, *dpart;
     RTB_TRY(w.alloc(&dmu, nm));
     RTB_TRY(w.alloc(&ds0, nm));
+    RTB_TRY(w.alloc(&dpart, rows * chunk));
     RTB_HIP(hipMemcpyAsync(dmu, mv, nm * sizeof(double), hipMemcpyHostToDevice, st));
     RTB_TRY(tmr.begin(RTB_STAGE_REDUCE));
     RTB_TRY(energy_cut_t0(st, m->dim, nx, ny, nz, n, dEv, dKv, dperm, dom, dmu, nm, eta, dpart, chunk, ds0));

@@ -244,10 +244,10 @@ int layer_partials(hipStream_t st, int n, size_t nk, const double* Z, const doub
 // band order (om [nk][n]; E [nk][n], Ki = Im K [nk][n][n], perm [nk][n]), and
 // the zero-width cut of every (cell, simplex, band) for the sorted mu (device,
 // n_mu) into out (device, n_mu), in launches of `chunk` chemical potentials
-// with partial [energy_cut_waves(...)][chunk] of scratch.
+// with partial [energy_cut_rows(.., n_mu)][chunk] of scratch.
 int energy_cut_omega(hipStream_t st, int n, size_t nk, const double* E, const double* Ki, const int* perm, double eta,
                      double* om);
-size_t energy_cut_waves(int dim, size_t nx, size_t ny, size_t nz, int n);
+size_t energy_cut_rows(int dim, size_t nx, size_t ny, size_t nz, int n, size_t n_mu);
 // Band tracking on the device for n <= kTrackDevMaxN: the walk of
 // energy_cut_track over the schedule of energy_cut_schedule, given as one
 // entry per vertex in level order (the vertex, its count of visited

@@ -195,6 +195,294 @@ __global__ void __launch_bounds__(256) cut_kernel(cut::View V, const double* __r
   }
 }
 
+// ---- many chemical potentials: lanes over mu ----
+// With a grid of chemical potentials finer than the bands' spread over a
+// simplex (the thermal convolution's: width / 10 apart) an item is cut at
+// hundreds of them, and the kernel above gathers its vertex data and adds up
+// a split band sum for each one.  Here a wave takes an item once: its lanes
+// copy E and Im K of the simplex's vertices, in ascending order of the band's
+// energy, to LDS and then take the item's sub-simplices of every chemical
+// potential, one per lane (1, 3 or 1 of a tetrahedron with one, two or three
+// vertices below mu, 1 or 2 of a triangle), each lane running the whole band
+// sums of its quadrature points from broadcast LDS reads.  The sub-simplices
+// of a mu are added in a fixed order, items follow each other in a fixed order
+// within a wave, a wave's sums are per mu, and the full items enter as steps
+// (one value at their first full mu, summed up at the end), so the result
+// does not depend on scheduling.
+// Bound: FP64 vector issue of the band sums.  20 x 18 x 16 cells of 5 simplices
+// and 12 bands, 2985 chemical potentials: 7.7 ms (294 ms by the kernel above).
+constexpr int kCutMu = 256;  // chemical potentials per wave (their sums sit in LDS), blocks of them in grid.y
+
+// LDS of a wave (doubles): sums and steps per mu, a sub-simplex value each,
+// then E and Im K [n][NV]
+__host__ __device__ inline size_t cut_mu_wave_doubles(int n, int nv) {
+  return static_cast<size_t>(2 + (nv - 1)) * kCutMu + 2 * static_cast<size_t>(n) * nv;
+}
+
+// The vertices of sub-simplex kind `kind` as sorted vertex pairs (p, q), four
+// bits each (p | q << 2), vertex k at bits 4k: the point of edge p-q on the
+// mu plane, or vertex p itself for p = q (clip_triangle, energy_cut.rs:1120-1169;
+// tetrahedron_occupied_hybrid, energy_cut.rs:1529-1640, where kind 4 is the
+// unoccupied corner).
+__device__ constexpr unsigned sub_code(int p0, int q0, int p1, int q1, int p2, int q2, int p3, int q3) {
+  return static_cast<unsigned>((p0 | q0 << 2) | (p1 | q1 << 2) << 4 | (p2 | q2 << 2) << 8 | (p3 | q3 << 2) << 12);
+}
+template <int NV>
+__device__ inline unsigned sub_vertices(int kind) {
+  if constexpr (NV == 4) {
+    constexpr unsigned k0 = sub_code(0, 0, 0, 1, 0, 2, 0, 3), k1 = sub_code(0, 0, 1, 1, 0, 2, 1, 3),
+                       k2 = sub_code(0, 0, 0, 2, 0, 3, 1, 3), k3 = sub_code(1, 1, 1, 2, 1, 3, 0, 2),
+                       k4 = sub_code(3, 3, 0, 3, 1, 3, 2, 3);
+    return kind == 0 ? k0 : (kind == 1 ? k1 : (kind == 2 ? k2 : (kind == 3 ? k3 : k4)));
+  } else {
+    constexpr unsigned k0 = sub_code(0, 0, 0, 1, 0, 2, 0, 0), k1 = sub_code(0, 0, 1, 1, 0, 2, 0, 0),
+                       k2 = sub_code(1, 1, 0, 2, 1, 2, 0, 0);
+    return kind == 0 ? k0 : (kind == 1 ? k1 : k2);
+  }
+}
+
+template <int DIM>
+__global__ void __launch_bounds__(256) cut_mu_kernel(cut::View V, const double* __restrict__ om, size_t nx, size_t ny,
+                                                     size_t nz, const double* __restrict__ mu, int mu_all, double eta,
+                                                     double* __restrict__ partial) {
+  constexpr int S = DIM == 2 ? 4 : 5;
+  constexpr int NV = DIM + 1;
+  extern __shared__ double smem[];
+  const int n = V.n;
+  const int mu0 = blockIdx.y * kCutMu;
+  const int n_mu = mu_all - mu0 < kCutMu ? mu_all - mu0 : kCutMu;
+  mu += mu0;
+  partial += mu0;  // rows of mu_all values
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  double* acc = smem + wave * cut_mu_wave_doubles(n, NV);  // [kCutMu] cut items per mu
+  double* step = acc + kCutMu;                             // [kCutMu] full items by their first full mu
+  double* sub = step + kCutMu;                             // [DIM * kCutMu] the item's sub-simplices
+  double* sE = sub + DIM * kCutMu;                         // [n][NV]
+  double* sK = sE + n * NV;
+  const size_t w = blockIdx.x * 4ull + wave, nw = gridDim.x * 4ull;
+  const size_t total = nx * ny * nz * S * static_cast<size_t>(n);
+  for (int i = lane; i < kCutMu; i += 64) {
+    acc[i] = 0.0;
+    step[i] = 0.0;
+  }
+  GpuTeam tm;
+  tm.wave_sync();
+  // first index in [a, b) with mu above x (or mu >= x when !above)
+  const auto first = [&](int a, int b, double x, bool above) {
+    while (a < b) {
+      const int c = (a + b) / 2;
+      const double m = mu[c];
+      if (above ? m <= x : m < x)
+        a = c + 1;
+      else
+        b = c;
+    }
+    return a;
+  };
+  const double eta2 = eta * eta;
+  for (size_t g0 = w * 64; g0 < total; g0 += nw * 64) {
+    // lane = item g0 + lane: its first cut and first full mu (the partition
+    // points of the sorted mu: full from mu >= e_max - eps on, below that
+    // empty up to mu <= e_min + eps, the rest cut)
+    const size_t g = g0 + lane;
+    int lo = n_mu, hi = n_mu;
+    double full = 0.0;
+    if (g < total) {
+      Simplex<DIM> x;
+      load_simplex<DIM>(V, om, g, nx, ny, nz, x);
+      if (!(x.measure < cut::kEps)) {  // degenerate simplices of ragged meshes
+        double e_min = x.e_v[0], e_max = x.e_v[0], osum = x.om_v[0];
+        for (int q = 1; q < NV; ++q) {
+          e_min = cut::dmin(e_min, x.e_v[q]);
+          e_max = cut::dmax(e_max, x.e_v[q]);
+          osum += x.om_v[q];
+        }
+        full = x.scale * (x.measure * osum / static_cast<double>(NV));
+        hi = first(0, n_mu, e_max - cut::kEps, false);
+        lo = first(0, hi, e_min + cut::kEps, true);
+      }
+    }
+    // full items in item order
+    unsigned long long fm = __ballot(hi < n_mu);
+    while (fm) {
+      const int l = __builtin_ctzll(fm);
+      fm &= fm - 1;
+      const int h = __builtin_amdgcn_readlane(hi, l);
+      const double f = lane_value(full, l);
+      if (lane == 0) step[h] += f;
+    }
+    // cut items in item order
+    unsigned long long cm = __ballot(lo < hi);
+    while (cm) {
+      const int l = __builtin_ctzll(cm);
+      cm &= cm - 1;
+      const int a0 = __builtin_amdgcn_readlane(lo, l), a1 = __builtin_amdgcn_readlane(hi, l);
+      const double vfull = lane_value(full, l);
+      Simplex<DIM> y;
+      load_simplex<DIM>(V, om, g0 + l, nx, ny, nz, y);
+      // vertices by ascending energy, ties in vertex order (sort_idx)
+      size_t vs[NV];
+      double e[NV];
+#pragma unroll
+      for (int q = 0; q < NV; ++q) {
+        vs[q] = y.vs[q];
+        e[q] = y.e_v[q];
+      }
+#pragma unroll
+      for (int round = 0; round < NV; ++round)
+#pragma unroll
+        for (int i = round % 2; i + 1 < NV; i += 2)
+          if (e[i + 1] < e[i]) {
+            const double te = e[i];
+            e[i] = e[i + 1];
+            e[i + 1] = te;
+            const size_t tv = vs[i];
+            vs[i] = vs[i + 1];
+            vs[i + 1] = tv;
+          }
+      tm.wave_sync();  // the previous item's reads are done
+      for (int q = lane; q < n * NV; q += 64) {
+        const int m = q / NV, v = q - m * NV;
+        size_t vq = vs[0];
+#pragma unroll
+        for (int u = 1; u < NV; ++u) vq = u == v ? vs[u] : vq;
+        sE[q] = cut::band(V, vq, m);
+        sK[q] = cut::kim(V, vq, y.b, m);
+      }
+      tm.wave_sync();
+      const double measure = y.measure;
+      // units: one sub-simplex for the mu up to vertex 1's energy (i1), DIM of
+      // them up to the next (i2; in 2D the rest), one above
+      const int i1 = first(a0, a1, e[1] + cut::kEps, true);
+      const int i2 = DIM == 3 ? first(i1, a1, e[DIM - 1] + cut::kEps, true) : a1;
+      const int n1 = i1 - a0, n2 = i2 - i1;
+      const int units = n1 + DIM * n2 + (a1 - i2);
+      for (int u = lane; u < units; u += 64) {
+        int i, kind;
+        if (u < n1) {
+          i = a0 + u;
+          kind = 0;
+        } else if (u < n1 + DIM * n2) {
+          const int r = u - n1;
+          i = i1 + r / DIM;
+          kind = 1 + r % DIM;
+        } else {
+          i = i2 + (u - n1 - DIM * n2);
+          kind = 4;
+        }
+        const double m = mu[i];
+        const unsigned code = sub_vertices<NV>(kind);
+        double sb[NV][NV];  // barycentric vertices
+        double vol = measure;
+#pragma unroll
+        for (int k = 0; k < NV; ++k) {
+          const int p = (code >> (4 * k)) & 3, q = (code >> (4 * k + 2)) & 3;
+          const double ep = cut::pick<NV>(e, p), de = cut::pick<NV>(e, q) - ep;
+          double t = 0.5;
+          if (!(fabs(de) < cut::kEps)) {
+            t = (m - ep) / de;
+            t = t < 0.0 ? 0.0 : (t > 1.0 ? 1.0 : t);
+          }
+          if (p == q) t = 0.0;
+#pragma unroll
+          for (int d = 0; d < NV; ++d) sb[k][d] = p == d ? 1.0 - t : (q == d ? t : 0.0);
+          // |det| of the barycentric rows: the product of the edge vertices'
+          // weights at the vertex no other row of the kind has
+          if (p != q) {
+            const bool one_minus = DIM == 3 ? kind == 4 || (kind >= 2 && k == 3) : kind == 2 && k == 1;
+            vol *= one_minus ? 1.0 - t : t;
+          }
+        }
+        double val = 0.0;
+        if (!(vol < 1e-30)) {
+          // the degree-2 rule: lam_k = wb sum of the vertices + (wa - wb) vertex k
+          constexpr double wa = DIM == 3 ? cut::kTA : 2.0 / 3.0, wb = DIM == 3 ? cut::kTB : 1.0 / 6.0;
+          double lam[NV][NV], en[NV], im[NV];
+#pragma unroll
+          for (int d = 0; d < NV; ++d) {
+            double t = sb[0][d];
+#pragma unroll
+            for (int k = 1; k < NV; ++k) t += sb[k][d];
+            t *= wb;
+#pragma unroll
+            for (int k = 0; k < NV; ++k) lam[k][d] = fma(wa - wb, sb[k][d], t);
+          }
+#pragma unroll
+          for (int k = 0; k < NV; ++k) {
+            im[k] = 0.0;
+            en[k] = 0.0;
+#pragma unroll
+            for (int d = 0; d < NV; ++d) en[k] = fma(sE[y.b * NV + d], lam[k][d], en[k]);
+          }
+          for (int mb = 0; mb < n; ++mb) {
+            if (mb == y.b) continue;  // the same in every lane
+            double ev[NV], kv[NV];
+#pragma unroll
+            for (int d = 0; d < NV; ++d) {
+              ev[d] = sE[mb * NV + d];
+              kv[d] = sK[mb * NV + d];
+            }
+#pragma unroll
+            for (int k = 0; k < NV; ++k) {
+              double de = en[k], kk = 0.0;
+#pragma unroll
+              for (int d = 0; d < NV; ++d) {
+                de = fma(-ev[d], lam[k][d], de);
+                kk = fma(kv[d], lam[k][d], kk);
+              }
+              const double denom = fma(de, de, eta2);
+              // hardware reciprocal and two Newton steps; a division where
+              // those would leave the number range
+              double r = __builtin_amdgcn_rcp(denom);
+              r = fma(r, fma(-denom, r, 1.0), r);
+              r = fma(r, fma(-denom, r, 1.0), r);
+              if (!(denom < 1e300)) r = 1.0 / denom;
+              if (!(denom < 1e-30)) im[k] = fma(kk, r, im[k]);
+            }
+          }
+          constexpr double wq = 1.0 / NV;
+#pragma unroll
+          for (int k = 0; k < NV; ++k) val += vol * wq * (-2.0 * im[k]);
+        }
+        sub[u] = kind == 4 ? -val : val;
+      }
+      tm.wave_sync();
+      // the sub-simplices of each mu, in order
+      for (int i = a0 + lane; i < a1; i += 64) {
+        double r;
+        if (i < i1) {
+          r = sub[i - a0];
+        } else if (i < i2) {
+          const int u = n1 + DIM * (i - i1);
+          r = sub[u];
+#pragma unroll
+          for (int q = 1; q < DIM; ++q) r += sub[u + q];
+        } else {
+          r = sub[n1 + DIM * n2 + (i - i2)];
+        }
+        r *= y.scale;
+        if (i >= i2) r += vfull;  // the full simplex minus the corner above mu
+        acc[i] += r;
+      }
+    }
+  }
+  tm.wave_sync();
+  // out[i] = cut sums + the steps up to i, 64 at a time with a carry
+  double carry = 0.0;
+  for (int i0 = 0; i0 < n_mu; i0 += 64) {
+    const int i = i0 + lane;
+    double s = i < n_mu ? step[i] : 0.0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const double t = __shfl_up(s, o);
+      if (lane >= o) s += t;
+    }
+    s += carry;
+    if (i < n_mu) partial[w * mu_all + i] = acc[i] + s;
+    carry = lane_value(s, 63);
+  }
+}
+
 // ---- band tracking (global_band_track, tracking.rs:123-163) ----
 // One workgroup per vertex of a level: the squared overlaps of its scheduled
 // neighbours (rows in the neighbour's tracked order) summed in neighbour
@@ -488,9 +776,27 @@ int energy_cut_omega(hipStream_t st, int n, size_t nk, const double* E, const do
   return RTB_OK;
 }
 
-size_t energy_cut_waves(int dim, size_t nx, size_t ny, size_t nz, int n) {
+static size_t energy_cut_waves(int dim, size_t nx, size_t ny, size_t nz, int n) {
   const size_t total = nx * ny * nz * (dim == 2 ? 4 : 5) * static_cast<size_t>(n);
   return (total + 255) / 256 * 4;
+}
+
+// Lanes over mu (cut_mu_kernel) from a full wave of chemical potentials on, if
+// there are at least 3/2 of them per mesh division: a band's spread over a cell
+// is about its width over the divisions, so below that an item is cut once or
+// not at all and most lanes idle.  Whole calls, mu over the band width, split
+// band sum against lanes over mu: n = 32 on 128 x 128, 64 mu 10.6 / 11.9 ms,
+// 128 mu 12.4 / 12.9, 256 mu 15.6 / 13.3; n = 96 on 24 x 24, 64 mu 11.8 / 8.3;
+// n = 12 on 20 x 18 x 16, 64 mu 6.7 / 2.2, 512 mu 48 / 3.5.
+static bool lanes_over_mu(size_t nx, size_t ny, size_t nz, size_t n_mu) {
+  return n_mu >= 64 && 2 * n_mu >= 3 * std::max(nx, std::max(ny, nz));
+}
+// partial rows (waves); with lanes over mu a wave covers one or more groups of
+// 64 items, so that the rows stay few
+constexpr size_t kCutMuRows = 8192;
+size_t energy_cut_rows(int dim, size_t nx, size_t ny, size_t nz, int n, size_t n_mu) {
+  const size_t waves = energy_cut_waves(dim, nx, ny, nz, n);
+  return lanes_over_mu(nx, ny, nz, n_mu) ? std::min(waves, kCutMuRows) : waves;
 }
 
 namespace {
@@ -529,6 +835,21 @@ int energy_cut_t0(hipStream_t st, int dim, size_t nx, size_t ny, size_t nz, int 
   const size_t waves = energy_cut_waves(dim, nx, ny, nz, n);
   const unsigned blocks = static_cast<unsigned>(waves / 4);
   const cut::View V{n, E, Ki, 1, perm};
+  if (lanes_over_mu(nx, ny, nz, n_mu)) {
+    const size_t rows = energy_cut_rows(dim, nx, ny, nz, n, n_mu);
+    const size_t smem = 4 * cut_mu_wave_doubles(n, dim + 1) * sizeof(double);
+    for (size_t m0 = 0; m0 < n_mu; m0 += chunk) {
+      const int c = static_cast<int>(std::min(chunk, n_mu - m0));
+      const dim3 grid(static_cast<unsigned>(rows / 4), static_cast<unsigned>((c + kCutMu - 1) / kCutMu));
+      if (dim == 2)
+        hipLaunchKernelGGL(cut_mu_kernel<2>, grid, dim3(256), smem, st, V, om, nx, ny, nz, mu + m0, c, eta, partial);
+      else
+        hipLaunchKernelGGL(cut_mu_kernel<3>, grid, dim3(256), smem, st, V, om, nx, ny, nz, mu + m0, c, eta, partial);
+      RTB_HIP(hipGetLastError());
+      RTB_TRY(column_sums(st, partial, rows, c, out + m0));
+    }
+    return RTB_OK;
+  }
   for (size_t m0 = 0; m0 < n_mu; m0 += chunk) {
     const int c = static_cast<int>(std::min(chunk, n_mu - m0));
     RTB_TRY(launch_cut(st, dim, n, blocks, V, om, nx, ny, nz, mu + m0, c, eta, partial));
@@ -538,6 +859,12 @@ int energy_cut_t0(hipStream_t st, int dim, size_t nx, size_t ny, size_t nz, int 
 }
 
 int energy_cut_track_smem_limits() {
+  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cut_mu_kernel<2>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              static_cast<int>(4 * cut_mu_wave_doubles(kTrackDevMaxN, 3) * sizeof(double))));
+  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&cut_mu_kernel<3>),
+                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                              static_cast<int>(4 * cut_mu_wave_doubles(kTrackDevMaxN, 4) * sizeof(double))));
   RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&track_kernel<true>),
                               hipFuncAttributeMaxDynamicSharedMemorySize,
                               static_cast<int>(track_smem(kTrackLdsMaxN))));

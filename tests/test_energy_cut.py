@@ -672,3 +672,27 @@ def test_gpu_n136_two_stage_vs_host_part():
     p = ra.Parameters.rank2(mesh, [1.0, 0.0], [0.0, 1.0], mu, eta=0.05, integration="EnergyCut")
     got = m.hall_conductivity(p).conductivity
     np.testing.assert_allclose(got, ref, rtol=0, atol=1e-8 * np.abs(ref).max())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dim,n,mesh,n_mu", [(2, 2, (9, 7), 64), (2, 33, (5, 6), 65), (2, 130, (3, 3), 129),
+                                             (2, 5, (1, 6), 300), (3, 12, (4, 5, 3), 513), (3, 65, (3, 2, 2), 70),
+                                             (3, 3, (3, 1, 4), 1300)])
+def test_gpu_many_chemical_potentials_equal_few(dim, n, mesh, n_mu):
+    """Calls with at least 64 chemical potentials on these meshes put the lanes
+    over mu, calls with fewer over the band sum: the same cut of the same items, equal to
+    rounding (two orders of the same FP64 sums, n * cells terms)."""
+    from rustb_amd.model import synth_model
+
+    m = synth_model(1 if dim == 3 else 3, dim, False, n, 1, 90 + n, scale=0.5, decay=1.0,
+                    n_R_target=0 if dim == 3 else 9)
+    w = 1.5 * math.sqrt(n)
+    mu = np.linspace(-w, w, n_mu)
+    d = np.eye(dim)[:2]
+    p = ra.Parameters(kmesh=mesh, direction=d, mu=mu, eta=0.02, integration="EnergyCut")
+    got = m.hall_conductivity(p).conductivity
+    ref = np.concatenate([m.hall_conductivity(ra.Parameters(kmesh=mesh, direction=d, mu=mu[i:i + 40], eta=0.02,
+                                                            integration="EnergyCut")).conductivity
+                          for i in range(0, n_mu, 40)])
+    assert np.abs(ref).max() > 0 or 1 in mesh
+    np.testing.assert_allclose(got, ref, rtol=0, atol=1e-11 * max(np.abs(ref).max(), 1e-3))
