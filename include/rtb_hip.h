@@ -407,7 +407,9 @@ const char* rtb_last_error(void);
  *   RTB_STAGE_KUBO       spin current and the Omega band sum
  *   RTB_STAGE_REDUCE     mesh points, occupation/DOS reductions, copies
  *   RTB_STAGE_TOTAL      first to last event of the call
- * ms[] in milliseconds; launches[] kernel launches per stage; flop[] the
+ * ms[] in milliseconds; launches[] kernel launches per stage (for the two
+ * product stages the products: a kernel that forms several counts each, and
+ * what it does with them is in its time); flop[] the
  * algorithmic floating-point operations of those launches where the stage
  * has a closed form (complex product 8 n^3, Hermitian product 4 n^2 (n+1),
  * tridiagonalisation 16/3 n^3, back-transformation 8 n^3; 0 otherwise);

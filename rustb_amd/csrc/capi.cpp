@@ -33,6 +33,7 @@ int prepare(const rtb_model* m) {
     g_smem_rc = mesh_set_smem_limits();
     if (g_smem_rc == RTB_OK) g_smem_rc = eigh_set_smem_limits();
     if (g_smem_rc == RTB_OK) g_smem_rc = energy_cut_track_smem_limits();
+    if (g_smem_rc == RTB_OK) g_smem_rc = col_set_smem_limits();
   });
   return g_smem_rc;
 }
@@ -388,6 +389,14 @@ int kubo_chunk(hipStream_t st, Timer& tmr, const rtb_model* m, size_t K, const d
       Ma = J;
       sMa = n2;
     }
+    if (n <= kMaxEighN) {
+      // the adjoint of A, then B and the band sum with it
+      RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
+      RTB_TRY(col_project_adjoint(st, n, K, Ma, sMa, Z, zscale, C));
+      RTB_TRY(col_kubo_exact(st, n, K, V + n2 * 2, 2 * n2, Z, zscale, C, E, eta, omega, metric, nullptr));
+      RTB_TRY(tmr.end(4, 4 * flop_zgemm(n, K), 4 * mflop_col(n, K)));
+      return RTB_OK;
+    }
     RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
     RTB_TRY(zgemm_batched(st, n, K, Ma, sMa, false, Z, n2, T1, n2));
     RTB_TRY(zgemm_batched_scaled(st, n, K, Z, n2, true, T1, n2, C, n2, false, zscale));
@@ -408,6 +417,12 @@ int kubo_chunk(hipStream_t st, Timer& tmr, const rtb_model* m, size_t K, const d
     RTB_TRY(spin_current(st, m->norb, K, spin_dir, V, 2 * n2 * 2, V + n2 * 2, J));
     RTB_TRY(tmr.end(1));
     M = J;
+  }
+  if (n <= kMaxEighN) {
+    RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
+    RTB_TRY(col_kubo(st, n, K, M, Z, zscale, E, eta, omega));
+    RTB_TRY(tmr.end(2, 2 * flop_zgemm(n, K), 2 * mflop_col(n, K)));
+    return RTB_OK;
   }
   RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
   // C = U^H M U for the unit eigenvectors U = Z diag(zscale) (zscale null: Z
@@ -441,6 +456,20 @@ int dipole_chunk(hipStream_t st, Timer& tmr, const rtb_model* m, size_t K, const
     Ma = J;
     sMa = n2;
   }
+  if (n <= kMaxEighN) {
+    // the adjoint of A1, then A2 and A3 with their band sums; their diagonals
+    // into T1
+    double *d2 = T1, *d3 = T1 + K * n;
+    RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
+    RTB_TRY(col_project_adjoint(st, n, K, Ma, sMa, Z, zscale, A1));
+    RTB_TRY(col_kubo_exact(st, n, K, V + n2 * 2, 3 * n2, Z, zscale, A1, E, eta, om1, nullptr, d2));
+    RTB_TRY(col_kubo_exact(st, n, K, V + n2 * 4, 3 * n2, Z, zscale, A1, E, eta, om2, nullptr, d3));
+    RTB_TRY(tmr.end(6, 6 * flop_zgemm(n, K), 6 * mflop_col(n, K)));
+    RTB_TRY(tmr.begin(RTB_STAGE_KUBO));
+    RTB_TRY(dipole_combine(st, n, K, d2, d3, n, 1, om1, om2, sym, kern));
+    RTB_TRY(tmr.end(1));
+    return RTB_OK;
+  }
   RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
   RTB_TRY(zgemm_batched(st, n, K, Ma, sMa, false, Z, n2, T1, n2));
   RTB_TRY(zgemm_batched_scaled(st, n, K, Z, n2, true, T1, n2, A1, n2, false, zscale));
@@ -452,7 +481,7 @@ int dipole_chunk(hipStream_t st, Timer& tmr, const rtb_model* m, size_t K, const
   RTB_TRY(tmr.begin(RTB_STAGE_KUBO));
   RTB_TRY(kubo_omega_exact(st, n, K, A1, A2, E, eta, om1, nullptr));
   if (sym) RTB_TRY(kubo_omega_exact(st, n, K, A1, A3, E, eta, om2, nullptr));
-  RTB_TRY(dipole_combine(st, n, K, A2, A3, om1, om2, sym, kern));
+  RTB_TRY(dipole_combine(st, n, K, A2, A3, 2 * n2, 2 * (static_cast<size_t>(n) + 1), om1, om2, sym, kern));
   RTB_TRY(tmr.end(sym ? 3 : 2));
   return RTB_OK;
 }
@@ -1557,6 +1586,13 @@ int rtb_hall_energy_cut(const rtb_model* m, const size_t* kmesh, const double* m
       Ma = dJ;
       sMa = n2;
     }
+    if (n <= kMaxEighN) {
+      RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
+      RTB_TRY(col_project_adjoint(st, n, c, Ma, sMa, Zc, nullptr, A));
+      RTB_TRY(col_im_k(st, n, c, dV + n2 * 2, 2 * n2, Zc, A, dKv + k0 * n2));
+      RTB_TRY(tmr.end(4, 4 * flop_zgemm(n, c), 4 * mflop_col(n, c)));
+      continue;
+    }
     RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
     RTB_TRY(zgemm_batched(st, n, c, Ma, sMa, false, Zc, n2, T1, n2));
     RTB_TRY(zgemm_batched(st, n, c, Zc, n2, true, T1, n2, A, n2));
@@ -1573,6 +1609,12 @@ int rtb_hall_energy_cut(const rtb_model* m, const size_t* kmesh, const double* m
   for (int ax = 0; ax < 3; ++ax) {
     for (size_t i0 = 0; i0 < cnt_ax[ax]; i0 += piece) {
       const size_t c = std::min(piece, cnt_ax[ax] - i0);
+      if (n <= kMaxEighN) {
+        RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
+        RTB_TRY(col_overlap2(st, n, c, dU + i0 * n2 * 2, dU + (i0 + step[ax]) * n2 * 2, dOv[ax] + i0 * n2));
+        RTB_TRY(tmr.end(1, flop_zgemm(n, c), mflop_col(n, c)));
+        continue;
+      }
       RTB_TRY(tmr.begin(RTB_STAGE_GEMM64));
       RTB_TRY(zgemm_batched(st, n, c, dU + i0 * n2 * 2, n2, true, dU + (i0 + step[ax]) * n2 * 2, n2, T1, n2));
       RTB_TRY(tmr.end(1, flop_zgemm(n, c), mflop_zgemm(n, c, false)));

@@ -201,6 +201,27 @@ int zgemm_batched(hipStream_t st, int n, size_t nb, const double* A, size_t sA, 
 int zgemm_batched_scaled(hipStream_t st, int n, size_t nb, const double* A, size_t sA, bool conj_a, const double* B,
                          size_t sB, double* C, size_t sC, bool herm, const double* s);
 
+// ---- products of one k-point kept on chip, n <= 128 (colprod.hip) ----
+// M, X: [nk] matrices at complex stride sX (M: n^2); Z: [nk][n][n] columns;
+// sc: [nk][n] scales of Z's columns (U = Z diag(sc)), or null.
+// Omega [nk][n] of the one-product band sum of U^H M U (M = A + i B operators).
+int col_kubo(hipStream_t st, int n, size_t nk, const double* M, const double* Z, const double* sc, const double* E,
+             double eta, double* omega);
+// P = U^H X^H U ([nk][n][n]): conj(P_ji) = (U^H X U)_ij.
+int col_project_adjoint(hipStream_t st, int n, size_t nk, const double* X, size_t sX, const double* Z,
+                        const double* sc, double* P);
+// With P of the first operator A and B = U^H X U: Omega_n = sum_{m != n} -2
+// Im(A_nm B_mn) / ((E_n - E_m)^2 + eta^2), optionally the metric's real part
+// and diag = Re B_nn.
+int col_kubo_exact(hipStream_t st, int n, size_t nk, const double* X, size_t sX, const double* Z, const double* sc,
+                   const double* P, const double* E, double eta, double* omega, double* metric, double* diag);
+// EnergyCut vertex kernel Im(A_ij B_ji) ([nk][n][n] real), B = Z^H X Z.
+int col_im_k(hipStream_t st, int n, size_t nk, const double* X, size_t sX, const double* Z, const double* P,
+             double* Ki);
+// out = |Ui^H Uj|^2 elementwise ([nk][n][n] real).
+int col_overlap2(hipStream_t st, int n, size_t nk, const double* Ui, const double* Uj, double* out);
+int col_set_smem_limits();
+
 // ---- Kubo band sum, reductions, DOS (kubo.hip) ----
 // J = (S v + v S) / 2 for the spin matrix S = sigma/2 (x) I (helpers.rs:11-39);
 // with w (stride v_stride like v) the output is J + i w.
@@ -224,9 +245,10 @@ int occupied_sum(hipStream_t st, int n, size_t nk, const double* omega, const do
 int hall_partials(hipStream_t st, int n, size_t nk, const double* omega, const double* E,
                   const double* mu, int n_mu, double T, double* partial, int n_blk, bool deriv = false);
 // Berry curvature dipole kernel per band: out = om1 * Re(A3_nn), or with sym
-// (om1 * Re(A3_nn) + om2 * Re(A2_nn)) / 2 (A2, A3: [nk][n][n], om: [nk][n]).
-int dipole_combine(hipStream_t st, int n, size_t nk, const double* A2, const double* A3, const double* om1,
-                   const double* om2, bool sym, double* out);
+// (om1 * Re(A3_nn) + om2 * Re(A2_nn)) / 2; Re(A_nn) of k-point k at
+// A[k * sk + n * sb] (om: [nk][n]).
+int dipole_combine(hipStream_t st, int n, size_t nk, const double* A2, const double* A3, size_t sk, size_t sb,
+                   const double* om1, const double* om2, bool sym, double* out);
 int hall_blocks(size_t nk);
 // out[k][m] = sum_n omega[k][n] f(E[k][n], mu_m, T) per k-point ([nk][n_mu]).
 int kterms(hipStream_t st, int n, size_t nk, const double* omega, const double* E, const double* mu, int n_mu,

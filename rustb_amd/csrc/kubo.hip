@@ -320,16 +320,14 @@ __global__ void __launch_bounds__(256) kubo_omega_exact_kernel(int n, const doub
 // response/nonlinear/mod.rs:140-162): Omega^{c,f1}_n Re(A3_nn), and with
 // `sym` the mean with Omega^{c,f2}_n Re(A2_nn) (FieldSymmetry::Symmetrized,
 // mod.rs:284-300); A2 = U^H v_f1 U, A3 = U^H v_f2 U.
-__global__ void dipole_combine_kernel(int n, size_t nk, const double2* __restrict__ A2,
-                                      const double2* __restrict__ A3, const double* __restrict__ om1,
+__global__ void dipole_combine_kernel(int n, size_t nk, const double* __restrict__ A2, const double* __restrict__ A3,
+                                      size_t sk, size_t sb, const double* __restrict__ om1,
                                       const double* __restrict__ om2, int sym, double* __restrict__ out) {
   const size_t g = blockIdx.x * 256ull + threadIdx.x;
   if (g >= nk * n) return;
-  const size_t k = g / n;
-  const int b = static_cast<int>(g % n);
-  const size_t d = k * n * n + static_cast<size_t>(b) * n + b;
-  const double first = om1[g] * A3[d].x;
-  out[g] = sym ? (first + om2[g] * A2[d].x) * 0.5 : first;
+  const size_t d = (g / n) * sk + (g % n) * sb;
+  const double first = om1[g] * A3[d];
+  out[g] = sym ? (first + om2[g] * A2[d]) * 0.5 : first;
 }
 
 }  // namespace
@@ -389,13 +387,12 @@ int layer_partials(hipStream_t st, int n, size_t nk, const double* Z, const doub
   return RTB_OK;
 }
 
-int dipole_combine(hipStream_t st, int n, size_t nk, const double* A2, const double* A3, const double* om1,
-                   const double* om2, bool sym, double* out) {
+int dipole_combine(hipStream_t st, int n, size_t nk, const double* A2, const double* A3, size_t sk, size_t sb,
+                   const double* om1, const double* om2, bool sym, double* out) {
   const size_t total = nk * n;
   if (total == 0) return RTB_OK;
   hipLaunchKernelGGL(dipole_combine_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0, st, n, nk,
-                     reinterpret_cast<const double2*>(A2), reinterpret_cast<const double2*>(A3), om1, om2,
-                     sym ? 1 : 0, out);
+                     A2, A3, sk, sb, om1, om2, sym ? 1 : 0, out);
   RTB_HIP(hipGetLastError());
   return RTB_OK;
 }

@@ -186,6 +186,11 @@ inline double mflop_zgemm(int n, size_t nb, bool herm) {
   const double tiles = herm ? side * (side + 1) / 2 : side * side;
   return tiles * 64.0 * 64.0 * kpad * 6.0 * static_cast<double>(nb);
 }
+// The same for a product of col_product_kernel (n <= 128): 16 x 16 tiles.
+inline double mflop_col(int n, size_t nb) {
+  const double N = ((n + 15) / 16) * 16.0;
+  return 6.0 * N * N * N * static_cast<double>(nb);
+}
 
 // EnergyCut Hall conductivity, host part (energy_cut.cpp).  Band tracking:
 // perm [nx ny][n] (band b of vertex i is raw band perm[i][b]) from the raw

@@ -1,0 +1,51 @@
+"""The on-chip products U^H X U at the edges of their 16-column tiles (every
+tile count from 1 to 8, sizes just below, at and above a tile), against the
+oracle: the term-by-term band sum (fp64, metric, spin current) and the
+one-product band sum (mixed)."""
+import numpy as np
+import pytest
+
+import rustb_amd as ra
+from oracle import oracle as O
+from rustb_amd.model import synth_model
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 2, 15, 16, 17, 32, 33, 47, 49, 64, 65, 81, 96, 97, 112, 113, 127, 128]
+
+
+def pair(n, spin=False):
+    m = synth_model(1, 3, spin, n // 2 if spin else n, 1, 300 + n, scale=0.5, decay=1.0)
+    return m, O.model_from_arrays(m.lat, m.orb, m.spin, m.hamR, m.ham)
+
+
+@pytest.mark.parametrize("n", EDGES)
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_omega_at_tile_edges(n, precision):
+    m, o = pair(n)
+    ks = np.random.default_rng(n).random((5, 3))
+    d = np.array([[1.0, 0.2, 0.0], [0.0, 1.0, -0.3]])
+    p = ra.Parameters(kmesh=(1, 1, 1), direction=d, mu=np.array([0.0]), eta=0.05, precision=precision)
+    om, E = m.berry_curvature_on(ks, p)
+    ob, Eb = O.berry_curvature_batch(o, ks, d, 0.05)
+    # Omega's error is an eigenvector's (rounding over the gap; fp64 ~1e-15,
+    # mixed ~1e-11 of the spectrum) times |v|^2 / eta^2: a few 1e2 of Omega's scale
+    tol = 1e-10 if precision == "fp64" else 1e-7
+    assert np.abs(E - Eb).max() < (1e-11 if precision == "fp64" else 1e-9)
+    assert np.abs(om - ob).max() <= tol * max(np.abs(ob).max(), 1e-3)
+
+
+@pytest.mark.parametrize("n", [2, 16, 34, 66, 98, 128])
+def test_spin_current_and_metric_at_tile_edges(n):
+    m, o = pair(n, spin=True)
+    ks = np.random.default_rng(n).random((4, 3))
+    d = np.eye(3)[:2]
+    p = ra.Parameters(kmesh=(1, 1, 1), direction=d, mu=np.array([0.0]), eta=0.05, spin="Y")
+    om, E = m.berry_curvature_on(ks, p)
+    ob, Eb = O.berry_curvature_batch(o, ks, d, 0.05, "Y")
+    assert np.abs(om - ob).max() <= 1e-10 * max(np.abs(ob).max(), 1e-3)
+    p.spin = None
+    r = m.quantum_geometry_on(ks, p)
+    for i, k in enumerate(ks):
+        g = O.quantum_geometry_at(o, k, d, 0.05)
+        assert np.abs(r.metric[i] - g[0]).max() <= 1e-10 * max(np.abs(g[0]).max(), 1e-3)
