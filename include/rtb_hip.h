@@ -402,7 +402,8 @@ const char* rtb_last_error(void);
  *   RTB_STAGE_BACKTRANS  eigenvector back-transformation kernel
  *   RTB_STAGE_GEMM64     FP64 matrix-core products (Kubo transforms and the
  *                        refinement products)
- *   RTB_STAGE_GEMM32     FP32 matrix-core correction products (refinement)
+ *   RTB_STAGE_GEMM32     FP32 matrix-core correction products (refinement;
+ *                        for nsta <= 128 their time is in RTB_STAGE_GEMM64)
  *   RTB_STAGE_REFINE     other refinement kernels (mixed form)
  *   RTB_STAGE_KUBO       spin current and the Omega band sum
  *   RTB_STAGE_REDUCE     mesh points, occupation/DOS reductions, copies

@@ -220,6 +220,8 @@ int col_im_k(hipStream_t st, int n, size_t nk, const double* X, size_t sX, const
              double* Ki);
 // out = |Ui^H Uj|^2 elementwise ([nk][n][n] real).
 int col_overlap2(hipStream_t st, int n, size_t nk, const double* Ui, const double* Uj, double* out);
+int col_refine(hipStream_t st, int n, size_t nk, const double* H, const float* Z, double* W1, double* W2, double* E,
+               double* scale, double* resid, double gap_rel);
 int col_set_smem_limits();
 
 // ---- Kubo band sum, reductions, DOS (kubo.hip) ----

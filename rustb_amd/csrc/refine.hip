@@ -36,7 +36,9 @@ __device__ inline double wave_sum(double x) {
 // the way.  Column j of Z (and of HZ = H Z) times scale[j] is the unit
 // vector; rotated columns are written unit.  Last, the k-point's check (see
 // RefineCheck).
-template <int NT>
+// kFromH: E, scale and the residuals (in `part`, [nk][n]) are there already
+// (col_refine), and HZ holds H: H z' is formed from it.
+template <int NT, bool kFromH>
 __global__ void __launch_bounds__(NT) cluster_rr_kernel(int n, double2* __restrict__ Z,
                                                         const double2* __restrict__ HZ,
                                                         const float2* __restrict__ F,
@@ -67,7 +69,10 @@ __global__ void __launch_bounds__(NT) cluster_rr_kernel(int n, double2* __restri
     __syncthreads();
     return m;
   };
-  {
+  if constexpr (kFromH) {
+    for (int j = tid; j < n; j += NT) s_res[j] = part[k * n + j];
+    __syncthreads();
+  } else {
     // Rayleigh quotients, column scales and residuals (against the
     // Ogita-Aishima quotients) from the per-tile sums of the correction
     // product's epilogue
@@ -103,20 +108,25 @@ __global__ void __launch_bounds__(NT) cluster_rr_kernel(int n, double2* __restri
       // (a run of more than kMaxCluster close eigenvalues is split; the
       // residuals of the columns at a split fail the check)
       if (c >= 2) {
-        // H z'_b = HZ (e_b + (F' - I)_b) for the cluster's columns, in FP64:
+        // H z'_b = HZ (e_b + (F' - I)_b) (kFromH: H z'_b) for the cluster's columns, in FP64:
         // one pass over row r of HZ for all of them
         for (int r = tid; r < n; r += NT) {
           const double2* hr = Hk + static_cast<size_t>(r) * n;
           double2 acc[kMaxCluster];
 #pragma unroll
-          for (int b = 0; b < kMaxCluster; ++b) acc[b] = b < c ? hr[j0 + b] : make_double2(0.0, 0.0);
+          for (int b = 0; b < kMaxCluster; ++b) acc[b] = b < c && !kFromH ? hr[j0 + b] : make_double2(0.0, 0.0);
           for (int q = 0; q < n; ++q) {
             const double2 h = hr[q];
             const float2* fq = Fk + static_cast<size_t>(q) * n + j0;
+            const double2* zq = Zk + static_cast<size_t>(q) * n + j0;
 #pragma unroll
             for (int b = 0; b < kMaxCluster; ++b)
               if (b < c) {
-                const float2 f = fq[b];
+                double2 f;
+                if constexpr (kFromH)
+                  f = zq[b];
+                else
+                  f = make_double2(fq[b].x, fq[b].y);
                 acc[b].x += h.x * f.x - h.y * f.y;
                 acc[b].y += h.x * f.y + h.y * f.x;
               }
@@ -319,8 +329,9 @@ int transpose_batched(hipStream_t st, int n, size_t nk, const double* Z, const d
 //   already ~1e-6 or smaller) stays below the FP64 level of the sums.  HZ'
 //   is never stored: its product's epilogue forms the Rayleigh sums
 //   Re(z'^H HZ') and z'^H z' per column, and the cluster kernel rebuilds
-//   H z' for the few columns inside clusters.
-// Buffers (each [nk][n][n] complex): H (consumed; F' - I in FP32), Z (in,
+//   H z' for the few columns inside clusters.  Up to n = 128 one kernel does
+//   all of it for a k-point (col_refine, its own form of the same step).
+// Buffers (each [nk][n][n] complex): H (above 128 consumed; F' - I in FP32), Z (in,
 // FP32), W1 (HZ), W3 (the Rayleigh sums); the refined eigenvectors are left in
 // W2 as columns that become unit vectors when multiplied by scale[k][j]
 // ([nk][n]; on entry the squared column norms of Z).
@@ -328,6 +339,33 @@ int refine_eigenpairs(hipStream_t st, Timer* tmr, int n, size_t nk, double* H, c
                       double* W2, double* W3, double* E, double* scale, double gap_rel, const RefineCheck& chk) {
   if (nk == 0) return RTB_OK;
   const size_t n2 = static_cast<size_t>(n) * n;
+  // a thread per row of the k-point's matrices
+  const int tiles = (n + 63) / 64;
+  double* part = W3;
+  auto rr = [&](auto kernel, int nt, const double* hz, const float* f) {
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(nk)), dim3(nt), 0, st, n, reinterpret_cast<double2*>(W2),
+                       reinterpret_cast<const double2*>(hz), reinterpret_cast<const float2*>(f), part, tiles, E,
+                       scale, gap_rel, chk);
+  };
+  if (n <= kMaxEighN) {
+    // the whole step in one kernel (R parked in W1), the residuals into W3;
+    // the corrections' time is in the FP64 products' stage
+    if (tmr) RTB_TRY(tmr->begin(RTB_STAGE_GEMM64));
+    RTB_TRY(col_refine(st, n, nk, H, Z, W1, W2, E, scale, part, gap_rel));
+    if (tmr) {
+      RTB_TRY(tmr->end(3, flop_zgemm(n, nk) + 2 * flop_zgemm_herm(n, nk), 2 * mflop_col(n, nk)));
+      RTB_TRY(tmr->begin(RTB_STAGE_GEMM32));
+      RTB_TRY(tmr->end(1, 2 * flop_zgemm(n, nk), 2 * mflop_col(n, nk)));
+      RTB_TRY(tmr->begin(RTB_STAGE_REFINE));
+    }
+    if (n <= 64)
+      rr(cluster_rr_kernel<64, true>, 64, H, nullptr);
+    else
+      rr(cluster_rr_kernel<128, true>, 128, H, nullptr);
+    RTB_HIP(hipGetLastError());
+    if (tmr) RTB_TRY(tmr->end(1));
+    return RTB_OK;
+  }
   // FP64 products: HZ, S = Z^H HZ, and G = Z^H Z consumed by its epilogue,
   // which writes F' - I (Z read from its exact FP32 storage; the exact
   // diagonal of G comes in `scale`)
@@ -342,24 +380,11 @@ int refine_eigenpairs(hipStream_t st, Timer* tmr, int n, size_t nk, double* H, c
   // Z' = Z + Z (F' - I) and HZ' = HZ + HZ (F' - I) in one kernel; HZ' is
   // consumed by its epilogue, which leaves the Rayleigh sums of the Z'
   // columns per 64-row tile in W3
-  const int tiles = (n + 63) / 64;
-  double* part = W3;
   if (tmr) RTB_TRY(tmr->begin(RTB_STAGE_GEMM32));
   RTB_TRY(zgemm_corrections_f32(st, n, nk, Z, W1, F, E, W2, part));  // both products, one pass over F
   if (tmr) RTB_TRY(tmr->end(1, 2 * flop_zgemm(n, nk), 2 * mflop_zgemm(n, nk, false)));
   if (tmr) RTB_TRY(tmr->begin(RTB_STAGE_REFINE));
-  // a thread per row of the k-point's matrices
-  auto rr = [&](auto kernel, int nt) {
-    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(nk)), dim3(nt), 0, st, n, reinterpret_cast<double2*>(W2),
-                       reinterpret_cast<const double2*>(W1), reinterpret_cast<const float2*>(F), part, tiles, E,
-                       scale, gap_rel, chk);
-  };
-  if (n <= 64)
-    rr(cluster_rr_kernel<64>, 64);
-  else if (n <= 128)
-    rr(cluster_rr_kernel<128>, 128);
-  else
-    rr(cluster_rr_kernel<256>, 256);
+  rr(cluster_rr_kernel<256, false>, 256, W1, F);
   RTB_HIP(hipGetLastError());
   if (tmr) RTB_TRY(tmr->end(1));
   return RTB_OK;
