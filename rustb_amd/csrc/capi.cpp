@@ -1819,7 +1819,7 @@ int rtb_dos(const rtb_model* m, const size_t* kmesh, double Emin, double Emax, s
   RTB_TRY(w.alloc(&dE, K * n));
   RTB_TRY(alloc_eig(w, n, K, false, eb));
   int total_blk = 0;
-  for (const Chunk& ch : chunks) total_blk += dos_blocks(ch.c * n);
+  for (const Chunk& ch : chunks) total_blk += dos_blocks(ch.c * n, static_cast<int>(En));
   double *dpart, *drho;
   RTB_TRY(w.alloc(&dpart, static_cast<size_t>(total_blk) * En));
   RTB_TRY(w.alloc(&drho, En));
@@ -1843,7 +1843,7 @@ int rtb_dos(const rtb_model* m, const size_t* kmesh, double Emin, double Emax, s
     RTB_TRY(eigh_launch_fp64(st, &tmr, n, c, dH, dE, false, eb.Vg, nullptr, nullptr, nullptr, eb.DE, false, eb.band));
     RTB_TRY(count_nonfinite(st, n, c, dE, ck.nonfinite));
     RTB_TRY(tmr.begin(RTB_STAGE_REDUCE));
-    const int nb = dos_blocks(c * n);
+    const int nb = dos_blocks(c * n, static_cast<int>(En));
     RTB_TRY(dos_partials(st, c * n, dE, Emin, step, static_cast<int>(En), sigma,
                          dpart + static_cast<size_t>(blk_off) * En, nb));
     RTB_TRY(tmr.end(1));

@@ -300,7 +300,7 @@ int abs2(hipStream_t st, size_t total, const double* z, double* x);
 // DOS partial sums: partial[blk][j] += sum_{eps in blk} g(E_j - eps)
 int dos_partials(hipStream_t st, size_t ne, const double* evals, double Emin, double dE, int En,
                  double sigma, double* partial, int n_blk);
-int dos_blocks(size_t ne);
+int dos_blocks(size_t ne, int En);
 // out[j] = scale * sum_blk partial[blk][j]
 int reduce_partials(hipStream_t st, const double* partial, int n_blk, int m, double scale, double* out);
 // out[j] = sum over n_rows rows of partial[r][j] (one workgroup per column, a

@@ -49,3 +49,28 @@ def test_spin_current_and_metric_at_tile_edges(n):
     for i, k in enumerate(ks):
         g = O.quantum_geometry_at(o, k, d, 0.05)
         assert np.abs(r.metric[i] - g[0]).max() <= 1e-10 * max(np.abs(g[0]).max(), 1e-3)
+
+
+@pytest.mark.parametrize("mesh,n_mu,T", [((1, 1), 1, 0.0), ((7, 9), 8, 300.0), ((8, 8), 9, 0.0), ((13, 5), 17, 900.0),
+                                         ((50, 41), 3, 300.0)])
+def test_hall_sums_at_block_edges(mesh, n_mu, T):
+    """The occupation sums in blocks of 64 k-points and 8 chemical potentials,
+    and the row sums above and below 32 blocks."""
+    m = synth_model(3, 2, False, 3, 1, 17, n_R_target=9)
+    o = O.model_from_arrays(m.lat, m.orb, m.spin, m.hamR, m.ham)
+    mu = np.linspace(-1.0, 1.3, n_mu)
+    p = ra.Parameters(kmesh=mesh, direction=np.eye(2), mu=mu, eta=0.05, T=np.array([T]))
+    got = m.hall_conductivity(p).conductivity
+    ref = O.hall_conductivity_direct(o, list(mesh), np.eye(2), mu, T, 0.05)
+    assert np.abs(got - ref).max() <= 1e-10 * max(np.abs(ref).max(), 1e-3)
+
+
+@pytest.mark.parametrize("mesh,En", [((1, 1), 1), ((5, 7), 256), ((33, 31), 257), ((200, 90), 801)])
+def test_dos_at_block_edges(mesh, En):
+    """The DOS in blocks of 64 to 2048 eigenvalues and 256 energies."""
+    m = ra.workloads.graphene()
+    o = O.model_from_arrays(m.lat, m.orb, m.spin, m.hamR, m.ham)
+    E, rho = m.dos(mesh, -4.0, 4.0, En, 0.05)
+    Er, rr = O.dos(o, list(mesh), -4.0, 4.0, En, 0.05)
+    # sums of nk positive terms in another order: nk eps of the result
+    assert np.abs(rho - rr).max() <= 1e-11 * max(np.abs(rr).max(), 1e-300)
