@@ -19,7 +19,9 @@
  *     for later calls until rtb_workspace_release() or process exit, so that
  *     repeated calls allocate nothing.  Concurrent large calls each hold
  *     their own block: an allocation the device cannot satisfy is
- *     RTB_ERR_DEVICE.  Host allocation is per call and proportional to the
+ *     RTB_ERR_DEVICE.  Small transfers go through 2 MB of pinned host memory
+ *     per concurrent call, kept until rtb_workspace_release() too.  Other host
+ *     allocation is per call and proportional to the
  *     outputs it stages (EnergyCut: the tracking walk's schedule, 32 bytes
  *     per k-point; its vertex data only under RTB_TRACK_HOST=1).
  */

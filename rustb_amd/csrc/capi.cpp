@@ -11,6 +11,7 @@
 
 #include "eigh.hpp"
 #include "pipeline.hpp"
+#include "staging.hpp"
 
 namespace rtb {
 
@@ -36,6 +37,24 @@ int prepare(const rtb_model* m) {
     if (g_smem_rc == RTB_OK) g_smem_rc = col_set_smem_limits();
   });
   return g_smem_rc;
+}
+
+// A call's transfers through its staging (staging.hpp), or as plain copies.
+static int to_device(hipStream_t st, Work& w, void* dst, const void* src, size_t bytes) {
+  if (w.stage) return w.stage->h2d(dst, src, bytes);
+  RTB_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
+  return RTB_OK;
+}
+static int to_host(hipStream_t st, Work& w, void* dst, const void* src, size_t bytes) {
+  if (w.stage) return w.stage->d2h(dst, src, bytes);
+  RTB_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+  return RTB_OK;
+}
+// waits for the stream; host targets of to_host hold their values afterwards
+static int wait_host(hipStream_t st, Work& w) {
+  if (w.stage) return w.stage->finish();
+  RTB_HIP(hipStreamSynchronize(st));
+  return RTB_OK;
 }
 
 bool finite(double x) { return std::isfinite(x); }
@@ -136,20 +155,10 @@ int upload_dirs(hipStream_t st, Work& w, const rtb_model* m, const double* dirs,
   double *dwR, *dwt;
   RTB_TRY(w.alloc(&dwR, wR.size()));
   RTB_TRY(w.alloc(&dwt, wt.size()));
-  RTB_HIP(hipMemcpyAsync(dwR, wR.data(), wR.size() * sizeof(double), hipMemcpyHostToDevice, st));
-  RTB_HIP(hipMemcpyAsync(dwt, wt.data(), wt.size() * sizeof(double), hipMemcpyHostToDevice, st));
+  RTB_TRY(to_device(st, w, dwR, wR.data(), wR.size() * sizeof(double)));
+  RTB_TRY(to_device(st, w, dwt, wt.data(), wt.size() * sizeof(double)));
   a.wR = dwR;
   a.wtau = dwt;
-  return RTB_OK;
-}
-
-// k rows of `dim` doubles -> device [nk][3] (zero padded)
-int upload_k(hipStream_t st, Work& w, int dim, const double* k, size_t nk, double** dk) {
-  std::vector<double> kp(nk * 3, 0.0);
-  for (size_t i = 0; i < nk; ++i)
-    for (int d = 0; d < dim; ++d) kp[i * 3 + d] = k[i * dim + d];
-  RTB_TRY(w.alloc(dk, kp.size()));
-  RTB_HIP(hipMemcpyAsync(*dk, kp.data(), kp.size() * sizeof(double), hipMemcpyHostToDevice, st));
   return RTB_OK;
 }
 
@@ -161,9 +170,19 @@ size_t workspace_budget() {
     const long long mb = std::atoll(env);
     if (mb > 0) return static_cast<size_t>(mb) << 20;
   }
-  size_t free_b = 0, total_b = 0;
-  if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || total_b == 0) return size_t(4) << 30;
-  return std::min(total_b / 8, size_t(32) << 30);
+  // the device's memory does not change: asked once per device (10 us)
+  static std::mutex mu;
+  static std::map<int, size_t> total;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return size_t(4) << 30;
+  std::lock_guard<std::mutex> lock(mu);
+  auto it = total.find(dev);
+  if (it == total.end()) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || total_b == 0) return size_t(4) << 30;
+    it = total.emplace(dev, total_b).first;
+  }
+  return std::min(it->second / 8, size_t(32) << 30);
 }
 
 size_t chunk_for(size_t nk, size_t per_k_bytes) {
@@ -275,16 +294,17 @@ template <typename KOf>
 int resolve_flagged(hipStream_t st, Work& w, Timer& tmr, const rtb_model* m, const FourierArgs& a, bool from_upper,
                     size_t c, KOf kof, Checks& ck, double* E, double* Zc, double* scale) {
   int cnt = 0;
-  RTB_HIP(hipMemcpyAsync(&cnt, ck.flag_count, sizeof(int), hipMemcpyDeviceToHost, st));
-  RTB_HIP(hipStreamSynchronize(st));
+  RTB_TRY(to_host(st, w, &cnt, ck.flag_count, sizeof(int)));
+  RTB_TRY(wait_host(st, w));
+  tmr.pause();
   if (cnt == 0) return RTB_OK;
   if (!ck.opt.fallback) {
     set_error("EigenvalueComputationFailed: the refined eigenpairs of %d k-point(s) fail the residual check", cnt);
     return RTB_ERR_EIGEN_FAILED;
   }
   std::vector<int> list(static_cast<size_t>(cnt));
-  RTB_HIP(hipMemcpyAsync(list.data(), ck.flag_list, list.size() * sizeof(int), hipMemcpyDeviceToHost, st));
-  RTB_HIP(hipStreamSynchronize(st));
+  RTB_TRY(to_host(st, w, list.data(), ck.flag_list, list.size() * sizeof(int)));
+  RTB_TRY(wait_host(st, w));
   const int n = m->nsta;
   const size_t n2 = static_cast<size_t>(n) * n;
   if (ck.cap == 0) {
@@ -303,7 +323,7 @@ int resolve_flagged(hipStream_t st, Work& w, Timer& tmr, const rtb_model* m, con
     const size_t bc = std::min(ck.cap, list.size() - b0);
     kp.assign(bc * 3, 0.0);
     for (size_t i = 0; i < bc; ++i) kof(static_cast<size_t>(list[b0 + i]), &kp[3 * i]);
-    RTB_HIP(hipMemcpyAsync(ck.dk, kp.data(), kp.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    RTB_TRY(to_device(st, w, ck.dk, kp.data(), kp.size() * sizeof(double)));
     RTB_TRY(tmr.begin(RTB_STAGE_FOURIER));
     RTB_TRY(fourier_dense(st, a0, ck.dk, bc, ck.H, nullptr));
     RTB_TRY(tmr.end(1));
@@ -317,23 +337,23 @@ int resolve_flagged(hipStream_t st, Work& w, Timer& tmr, const rtb_model* m, con
     RTB_TRY(count_nonfinite(st, n, bc, ck.E, ck.nonfinite));
     RTB_TRY(scatter_resolved(st, n, static_cast<int>(bc), ck.flag_list + b0, ck.E, ck.Z, E, Zc, scale));
     RTB_TRY(tmr.end(2));
-    RTB_HIP(hipStreamSynchronize(st));  // kp is refilled next
+    RTB_TRY(wait_host(st, w));  // kp is refilled next
   }
   RTB_TRY(zero_ints(st, ck.flag_count, 1));
   ck.resolved += list.size();
   return RTB_OK;
 }
 
-// End of a call: the largest refined residual and the re-solved count into
+// End of a call (waits for the stream): the largest refined residual and the re-solved count into
 // the stats; RTB_ERR_EIGEN_FAILED when an eigenvalue is not finite.
-int checks_finish(hipStream_t st, Checks& ck, Timer& tmr) {
-  int nf = 0;
-  unsigned long long mr = 0;
-  RTB_HIP(hipMemcpyAsync(&nf, ck.nonfinite, sizeof(int), hipMemcpyDeviceToHost, st));
-  RTB_HIP(hipMemcpyAsync(&mr, ck.max_res, sizeof(mr), hipMemcpyDeviceToHost, st));
-  RTB_HIP(hipStreamSynchronize(st));
+int checks_finish(hipStream_t st, Work& w, Checks& ck, Timer& tmr) {
+  int c[4] = {0, 0, 0, 0};  // flag count, non-finite count, bits of the largest residual
+  static_assert(sizeof(c) == 2 * sizeof(int) + sizeof(unsigned long long), "the counters' layout (checks_alloc)");
+  RTB_TRY(to_host(st, w, c, ck.flag_count, sizeof(c)));
+  RTB_TRY(wait_host(st, w));
+  const int nf = c[1];
   double r;
-  std::memcpy(&r, &mr, sizeof(r));
+  std::memcpy(&r, c + 2, sizeof(r));
   tmr.note_check(r, ck.resolved);
   if (nf > 0) {
     set_error("EigenvalueComputationFailed: the eigenvalues of %d k-point(s) are not finite", nf);
@@ -732,6 +752,8 @@ int rtb_gen_ham_batch(const rtb_model* m, const double* k, size_t nk, int gauge,
   RTB_TRY(lease.status());
   hipStream_t st = lease.stream();
   Work w(lease);
+  Staging stage(st);
+  w.stage = &stage;
   Timer tmr(lease);
   FourierArgs a;
   RTB_TRY(upload_dirs(st, w, m, dirs, n_proj, a));
@@ -756,7 +778,7 @@ int rtb_gen_ham_batch(const rtb_model* m, const double* k, size_t nk, int gauge,
     kp.assign(c * 3, 0.0);
     for (size_t i = 0; i < c; ++i)
       for (int d = 0; d < m->dim; ++d) kp[i * 3 + d] = k[(k0 + i) * m->dim + d];
-    RTB_HIP(hipMemcpyAsync(dk, kp.data(), kp.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    RTB_TRY(to_device(st, w, dk, kp.data(), kp.size() * sizeof(double)));
     RTB_TRY(tmr.begin(RTB_STAGE_FOURIER));
     RTB_TRY(fourier_dense(st, a, dk, c, dH, dV));
     RTB_TRY(tmr.end(1));
@@ -765,11 +787,11 @@ int rtb_gen_ham_batch(const rtb_model* m, const double* k, size_t nk, int gauge,
       RTB_TRY(rmatrix_velocity(st, a, m->d_rmat, dirs, dk, c, dH, dV, rproj, Rk, T1, T2));
       RTB_TRY(tmr.end(1));
     }
-    RTB_HIP(hipMemcpyAsync(H + k0 * n2 * 2, dH, c * n2 * 2 * sizeof(double), hipMemcpyDeviceToHost, st));
+    RTB_TRY(to_host(st, w, H + k0 * n2 * 2, dH, c * n2 * 2 * sizeof(double)));
     if (n_proj)
-      RTB_HIP(hipMemcpyAsync(V + k0 * n_proj * n2 * 2, dV, c * n_proj * n2 * 2 * sizeof(double),
-                             hipMemcpyDeviceToHost, st));
-    RTB_HIP(hipStreamSynchronize(st));
+      RTB_TRY(to_host(st, w, V + k0 * n_proj * n2 * 2, dV, c * n_proj * n2 * 2 * sizeof(double)));
+    RTB_TRY(wait_host(st, w));
+    tmr.pause();
   }
   RTB_TRY(tmr.collect(nk, n));
   return RTB_OK;
@@ -790,6 +812,8 @@ static int solve_impl(const rtb_model* m, const double* k, size_t nk, int precis
   RTB_TRY(lease.status());
   hipStream_t st = lease.stream();
   Work w(lease);
+  Staging stage(st);
+  w.stage = &stage;
   Timer tmr(lease);
   FourierArgs a;
   RTB_TRY(upload_dirs(st, w, m, nullptr, 0, a));
@@ -821,7 +845,7 @@ static int solve_impl(const rtb_model* m, const double* k, size_t nk, int precis
     kp.assign(c * 3, 0.0);
     for (size_t i = 0; i < c; ++i)
       for (int d = 0; d < m->dim; ++d) kp[i * 3 + d] = k[(k0 + i) * m->dim + d];
-    RTB_HIP(hipMemcpyAsync(dk, kp.data(), kp.size() * sizeof(double), hipMemcpyHostToDevice, st));
+    RTB_TRY(to_device(st, w, dk, kp.data(), kp.size() * sizeof(double)));
     RTB_TRY(tmr.begin(RTB_STAGE_FOURIER));
     RTB_TRY(fourier_dense(st, a, dk, c, dH, nullptr));
     RTB_TRY(tmr.end(1));
@@ -846,12 +870,14 @@ static int solve_impl(const rtb_model* m, const double* k, size_t nk, int precis
         RTB_TRY(tmr.end(1, flop_backtrans(n, c)));
       }
     }
-    RTB_HIP(hipMemcpyAsync(E + k0 * n, dE, c * n * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (vec)
-      RTB_HIP(hipMemcpyAsync(evec + k0 * n2 * 2, dZ, c * n2 * 2 * sizeof(double), hipMemcpyDeviceToHost, st));
-    RTB_HIP(hipStreamSynchronize(st));
+    RTB_TRY(to_host(st, w, E + k0 * n, dE, c * n * sizeof(double)));
+    if (vec) RTB_TRY(to_host(st, w, evec + k0 * n2 * 2, dZ, c * n2 * 2 * sizeof(double)));
+    if (k0 + K < nk) {  // the last chunk's outputs come with the counters
+      RTB_TRY(wait_host(st, w));
+      tmr.pause();
+    }
   }
-  RTB_TRY(checks_finish(st, ck, tmr));
+  RTB_TRY(checks_finish(st, w, ck, tmr));
   RTB_TRY(tmr.collect(nk, n));
   return RTB_OK;
 }
@@ -1136,14 +1162,15 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
   double* T1 = bb.kub;
   double* A = bb.kub + K * n2 * 2;
   double* B = bb.kub + K * n2 * 4;
-  if (j.mode == 2) RTB_HIP(hipMemcpyAsync(dmu, j.mu, j.n_mu * sizeof(double), hipMemcpyHostToDevice, st));
+  if (j.mode == 2) RTB_TRY(to_device(st, w, dmu, j.mu, j.n_mu * sizeof(double)));
   const size_t ml = j.n_mu * static_cast<size_t>(j.n_layers);
   if (j.n_layers > 0) {
-    RTB_HIP(hipMemcpyAsync(bb.dperm, j.layer_perm, sizeof(int) * n, hipMemcpyHostToDevice, st));
-    RTB_HIP(hipMemcpyAsync(bb.dbounds, j.layer_bounds, sizeof(int) * (j.n_layers + 1), hipMemcpyHostToDevice, st));
+    RTB_TRY(to_device(st, w, bb.dperm, j.layer_perm, sizeof(int) * n));
+    RTB_TRY(to_device(st, w, bb.dbounds, j.layer_bounds, sizeof(int) * (j.n_layers + 1)));
   }
   size_t chunk_no = 0;
   std::vector<double> kp;
+  std::vector<double> sums(j.mode == 2 ? j.n_mu : 0), msums(j.mode == 2 && j.geometry ? j.n_mu : 0);
   int blk_off = 0;
   for (const Chunk& ch : chunks) {
     const size_t k0 = ch.k0, c = ch.c;
@@ -1151,7 +1178,7 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
       kp.assign(c * 3, 0.0);
       for (size_t i = 0; i < c; ++i)
         for (int d = 0; d < m->dim; ++d) kp[i * 3 + d] = j.k[(k0 + i) * m->dim + d];
-      RTB_HIP(hipMemcpyAsync(dk, kp.data(), kp.size() * sizeof(double), hipMemcpyHostToDevice, st));
+      RTB_TRY(to_device(st, w, dk, kp.data(), kp.size() * sizeof(double)));
     }
     if (G) {
       RTB_TRY(tmr.begin(RTB_STAGE_FOURIER));
@@ -1216,14 +1243,13 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
     int l2 = 0;
     RTB_TRY(tmr.begin(RTB_STAGE_REDUCE));
     if (j.mode == 0) {
-      RTB_HIP(hipMemcpyAsync(j.omega + k0 * n, dOm, c * n * sizeof(double), hipMemcpyDeviceToHost, st));
-      RTB_HIP(hipMemcpyAsync(j.E + k0 * n, dE, c * n * sizeof(double), hipMemcpyDeviceToHost, st));
-      if (j.geometry)
-        RTB_HIP(hipMemcpyAsync(j.metric + k0 * n, dMet, c * n * sizeof(double), hipMemcpyDeviceToHost, st));
+      RTB_TRY(to_host(st, w, j.omega + k0 * n, dOm, c * n * sizeof(double)));
+      RTB_TRY(to_host(st, w, j.E + k0 * n, dE, c * n * sizeof(double)));
+      if (j.geometry) RTB_TRY(to_host(st, w, j.metric + k0 * n, dMet, c * n * sizeof(double)));
     } else if (j.mode == 1) {
       RTB_TRY(occupied_sum(st, n, c, dOm, dE, j.mu0, j.T, docc));
       ++l2;
-      RTB_HIP(hipMemcpyAsync(j.occ + k0, docc, c * sizeof(double), hipMemcpyDeviceToHost, st));
+      RTB_TRY(to_host(st, w, j.occ + k0, docc, c * sizeof(double)));
     } else {
       const int nb = hall_blocks(c);
       RTB_TRY(hall_partials(st, n, c, j.dipole ? dKern : dOm, dE, dmu, static_cast<int>(j.n_mu), j.T,
@@ -1244,7 +1270,10 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
       blk_off += nb;
     }
     RTB_TRY(tmr.end(l2));
-    if (j.mode != 2) RTB_HIP(hipStreamSynchronize(st));
+    if (j.mode != 2 && &ch != &chunks.back()) {  // the last chunk's outputs come with the counters
+      RTB_TRY(wait_host(st, w));
+      tmr.pause();
+    }
     ++chunk_no;
   }
   if (j.mode == 2) {
@@ -1252,23 +1281,23 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
     RTB_TRY(reduce_partials(st, dpart, total_blk, static_cast<int>(j.n_mu), 1.0, dsig));
     if (j.geometry) RTB_TRY(reduce_partials(st, dmpart, total_blk, static_cast<int>(j.n_mu), 1.0, dmsig));
     RTB_TRY(tmr.end(j.geometry ? 2 : 1));
-    std::vector<double> sums(j.n_mu), msums(j.geometry ? j.n_mu : 0);
-    RTB_HIP(hipMemcpyAsync(sums.data(), dsig, j.n_mu * sizeof(double), hipMemcpyDeviceToHost, st));
-    if (j.geometry)
-      RTB_HIP(hipMemcpyAsync(msums.data(), dmsig, j.n_mu * sizeof(double), hipMemcpyDeviceToHost, st));
-    RTB_HIP(hipStreamSynchronize(st));
+    RTB_TRY(to_host(st, w, sums.data(), dsig, j.n_mu * sizeof(double)));
+    if (j.geometry) RTB_TRY(to_host(st, w, msums.data(), dmsig, j.n_mu * sizeof(double)));
+    if (j.n_layers > 0) {
+      RTB_TRY(reduce_partials(st, bb.dlsum, static_cast<int>(chunks.size()), static_cast<int>(ml), 1.0, bb.dlay));
+      RTB_TRY(to_host(st, w, j.sigma_layers, bb.dlay, ml * sizeof(double)));
+    }
+  }
+  const int rc = checks_finish(st, w, ck, tmr);  // waits for the sums
+  if (rc != RTB_OK && rc != RTB_ERR_EIGEN_FAILED) return rc;
+  if (j.mode == 2) {
     // sum / nk / det (response/linear/mod.rs:221; quantum_geometry.rs:219,234)
     for (size_t i = 0; i < j.n_mu; ++i) j.sigma[i] = sums[i] / static_cast<double>(j.nk) / m->det_lat;
     for (size_t i = 0; i < msums.size(); ++i) j.msum[i] = msums[i] / static_cast<double>(j.nk) / m->det_lat;
-    if (j.n_layers > 0) {
-      RTB_TRY(reduce_partials(st, bb.dlsum, static_cast<int>(chunks.size()), static_cast<int>(ml), 1.0, bb.dlay));
-      RTB_HIP(hipMemcpyAsync(j.sigma_layers, bb.dlay, ml * sizeof(double), hipMemcpyDeviceToHost, st));
-      RTB_HIP(hipStreamSynchronize(st));
+    if (j.n_layers > 0)
       for (size_t i = 0; i < ml; ++i) j.sigma_layers[i] /= static_cast<double>(j.nk) * m->det_lat;
-    }
   }
-  RTB_HIP(hipStreamSynchronize(st));
-  RTB_TRY(checks_finish(st, ck, tmr));
+  RTB_TRY(rc);
   RTB_TRY(tmr.collect(j.nk, n));
   return RTB_OK;
 }
@@ -1277,6 +1306,8 @@ static int berry_impl(const rtb_model* m, BerryJob& j) {
   Lease lease;
   RTB_TRY(lease.status());
   Work w(lease);
+  Staging stage(lease.stream());
+  w.stage = &stage;
   Timer tmr(lease);
   Exec ex;
   ex.st = lease.stream();
@@ -1501,6 +1532,8 @@ int rtb_hall_energy_cut(const rtb_model* m, const size_t* kmesh, const double* m
   RTB_TRY(lease.status());
   hipStream_t st = lease.stream();
   Work w(lease);
+  Staging stage(st);
+  w.stage = &stage;
   Timer tmr(lease);
   FourierArgs a;
   RTB_TRY(upload_dirs(st, w, m, dir, 2, a));
@@ -1554,8 +1587,8 @@ int rtb_hall_energy_cut(const rtb_model* m, const size_t* kmesh, const double* m
       for (int r = 0; r < 6; ++r) e.dep[r] = r < static_cast<int>(e.cnt) ? static_cast<unsigned>(ts.dep[v * 6 + r]) : 0u;
     }
     RTB_TRY(w.alloc(&sched, nk));
-    RTB_HIP(hipMemcpyAsync(sched, he.data(), nk * sizeof(TrackEntry), hipMemcpyHostToDevice, st));
-    RTB_HIP(hipStreamSynchronize(st));  // the host vector goes out of scope here
+    RTB_TRY(to_device(st, w, sched, he.data(), nk * sizeof(TrackEntry)));
+    RTB_TRY(wait_host(st, w));  // the host vector goes out of scope here
   }
   Checks ck;
   RTB_TRY(checks_init(st, w, 0, ck));
@@ -1680,15 +1713,15 @@ int rtb_hall_energy_cut(const rtb_model* m, const size_t* kmesh, const double* m
     RTB_TRY(w.alloc(&dmu, nm));
     RTB_TRY(w.alloc(&ds0, nm));
     RTB_TRY(w.alloc(&dpart, rows * chunk));
-    RTB_HIP(hipMemcpyAsync(dmu, mv, nm * sizeof(double), hipMemcpyHostToDevice, st));
+    RTB_TRY(to_device(st, w, dmu, mv, nm * sizeof(double)));
     RTB_TRY(tmr.begin(RTB_STAGE_REDUCE));
     RTB_TRY(energy_cut_t0(st, m->dim, nx, ny, nz, n, dEv, dKv, dperm, dom, dmu, nm, eta, dpart, chunk, ds0));
     RTB_TRY(tmr.end(static_cast<int>(2 * ((nm + chunk - 1) / chunk))));
-    RTB_HIP(hipMemcpyAsync(s0, ds0, nm * sizeof(double), hipMemcpyDeviceToHost, st));
-    RTB_HIP(hipStreamSynchronize(st));
+    RTB_TRY(to_host(st, w, s0, ds0, nm * sizeof(double)));
+    RTB_TRY(wait_host(st, w));
     return RTB_OK;
   }, sigma));
-  RTB_TRY(checks_finish(st, ck, tmr));
+  RTB_TRY(checks_finish(st, w, ck, tmr));
   RTB_TRY(tmr.collect(nk, n));
   for (size_t i = 0; i < n_mu; ++i) sigma[i] /= m->det_lat;  // linear/mod.rs:267
   return RTB_OK;
@@ -1802,6 +1835,8 @@ int rtb_dos(const rtb_model* m, const size_t* kmesh, double Emin, double Emax, s
   RTB_TRY(lease.status());
   hipStream_t st = lease.stream();
   Work w(lease);
+  Staging stage(st);
+  w.stage = &stage;
   Timer tmr(lease);
   FourierArgs a;
   RTB_TRY(upload_dirs(st, w, m, nullptr, 0, a));
@@ -1852,10 +1887,10 @@ int rtb_dos(const rtb_model* m, const size_t* kmesh, double Emin, double Emax, s
   RTB_TRY(tmr.begin(RTB_STAGE_REDUCE));
   RTB_TRY(reduce_partials(st, dpart, total_blk, static_cast<int>(En), 1.0, drho));
   RTB_TRY(tmr.end(1));
-  RTB_HIP(hipMemcpyAsync(rho, drho, En * sizeof(double), hipMemcpyDeviceToHost, st));
-  RTB_HIP(hipStreamSynchronize(st));
+  RTB_TRY(to_host(st, w, rho, drho, En * sizeof(double)));
+  const int rc = checks_finish(st, w, ck, tmr);  // waits for rho
   for (size_t i = 0; i < En; ++i) rho[i] /= static_cast<double>(nk);  // model_physics.rs:224
-  RTB_TRY(checks_finish(st, ck, tmr));
+  RTB_TRY(rc);
   RTB_TRY(tmr.collect(nk, n));
   return RTB_OK;
 }

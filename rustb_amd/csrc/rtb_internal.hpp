@@ -47,6 +47,9 @@ inline int fail(int code, const char* msg) {
 // default 4) hold a slot on one device at once; further callers wait.
 struct Slot;
 int max_concurrent_calls();
+// Run by rtb_workspace_release after the slots are freed (null: nothing).
+using ReleaseHook = void (*)();
+ReleaseHook& workspace_release_hook();
 class Lease {
  public:
   Lease();   // takes a slot on the current device (waits while all are busy)
@@ -68,8 +71,10 @@ class Lease {
 // from a leased slot's block (which grows when a call needs more) or from a
 // fixed buffer (no growth: a request beyond it is RTB_ERR_UNSUPPORTED).  A
 // fixed buffer with a null base only counts the bytes requested (sizing).
+class Staging;
 class Work {
  public:
+  Staging* stage = nullptr;  // the call's pinned staging, or null: pageable copies
   explicit Work(Lease& l);
   Work(void* base, size_t cap);
   Work(const Work&) = delete;
@@ -104,18 +109,27 @@ class Timer {
   int begin(int stage) {
     if (!lease_) return RTB_OK;
     Rec r{stage, nullptr, nullptr, 0, 0.0, 0.0};
-    RTB_TRY(lease_->event(2 * recs_.size(), &r.a));
+    // a stage starts where the one before it ended, unless the host waited or
+    // moved outputs in between (pause): half the events to record
+    if (open_ && !recs_.empty()) {
+      r.a = recs_.back().b;
+    } else {
+      RTB_TRY(lease_->event(2 * recs_.size(), &r.a));
+      RTB_HIP(hipEventRecord(r.a, st_));
+    }
     RTB_TRY(lease_->event(2 * recs_.size() + 1, &r.b));
-    RTB_HIP(hipEventRecord(r.a, st_));
     recs_.push_back(r);
     return RTB_OK;
   }
+  // the next stage records its own start
+  void pause() { open_ = false; }
   int end(int launches, double flop = 0.0, double mflop = 0.0) {
     if (!lease_) return RTB_OK;
     recs_.back().launches = launches;
     recs_.back().flop = flop;
     recs_.back().mflop = mflop;
     RTB_HIP(hipEventRecord(recs_.back().b, st_));
+    open_ = true;
     return RTB_OK;
   }
   // the eigenpair checks of the call: largest refined residual (eV) and the
@@ -169,6 +183,7 @@ class Timer {
   Lease* lease_ = nullptr;
   hipStream_t st_ = nullptr;
   std::vector<Rec> recs_;
+  bool open_ = false;  // the last record's end event is the stream's last work
   double max_res_ = 0.0;
   size_t resolved_ = 0;
 };

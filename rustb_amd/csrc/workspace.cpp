@@ -42,6 +42,11 @@ size_t round_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 }  // namespace
 
+ReleaseHook& workspace_release_hook() {
+  static ReleaseHook hook = nullptr;
+  return hook;
+}
+
 int max_concurrent_calls() {
   if (const char* env = std::getenv("RTB_MAX_CONCURRENT_CALLS")) {
     const int v = std::atoi(env);
@@ -184,6 +189,7 @@ int rtb_workspace_release(void) {
     (void)hipStreamDestroy(s->stream);
     delete s;
   }
+  if (workspace_release_hook()) workspace_release_hook()();
   return RTB_OK;
 }
 
