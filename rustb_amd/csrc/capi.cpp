@@ -125,6 +125,8 @@ int upload_dirs(hipStream_t st, Work& w, const rtb_model* m, const double* dirs,
   a.ham = m->d_ham;
   a.R = m->d_R;
   a.tau = m->d_tau;
+  a.npair = m->npair;
+  a.pairs = m->d_pairs;
   a.wR = nullptr;
   a.wtau = nullptr;
   if (np == 0) return RTB_OK;
@@ -557,6 +559,30 @@ int upload_pageable(void* dst, const void* src, size_t bytes) {
   return rc;
 }
 
+// Every stored R once: (r, the index of -R) for the first of two, (r, -1) where
+// -R is not stored or is R itself; a repeated R stands by itself.
+std::vector<int> pair_table(int dim, int n_R, const int64_t* hamR) {
+  std::map<std::vector<int64_t>, std::vector<int>> waiting;  // R -> stored, unpaired indices
+  std::vector<int> partner(n_R, -1), out;
+  std::vector<char> second(n_R, 0);
+  for (int r = 0; r < n_R; ++r) {
+    std::vector<int64_t> R(hamR + r * dim, hamR + (r + 1) * dim), neg(R);
+    for (int64_t& x : neg) x = -x;
+    if (neg == R) continue;
+    auto it = waiting.find(neg);
+    if (it != waiting.end() && !it->second.empty()) {
+      partner[it->second.back()] = r;
+      second[r] = 1;
+      it->second.pop_back();
+    } else {
+      waiting[R].push_back(r);
+    }
+  }
+  for (int r = 0; r < n_R; ++r)
+    if (!second[r]) out.insert(out.end(), {r, partner[r]});
+  return out;
+}
+
 // ham[-R] == ham[R]^H exactly for every stored R (the builder's storage, by
 // construction); models read from files are Hermitian only to their printed
 // precision.  Decides whether the velocity operators may be combined into
@@ -699,14 +725,18 @@ int rtb_model_create(int dim, int spin, int norb, int n_R, const int64_t* hamR, 
       tauc[o * 3 + d] = s;
     }
   }
+  const std::vector<int> pairs = pair_table(dim, n_R, hamR);
+  m->npair = static_cast<int>(pairs.size() / 2);
   if (hipMalloc(&m->d_ham, sizeof(double) * 2 * n2 * n_R) != hipSuccess ||
+      hipMalloc(&m->d_pairs, sizeof(int) * pairs.size()) != hipSuccess ||
       hipMalloc(&m->d_R, sizeof(double) * R.size()) != hipSuccess ||
       hipMalloc(&m->d_Rcart, sizeof(double) * Rc.size()) != hipSuccess ||
       hipMalloc(&m->d_tau, sizeof(double) * tau.size()) != hipSuccess ||
       hipMalloc(&m->d_taucart, sizeof(double) * tauc.size()) != hipSuccess)
     return cleanup(fail(RTB_ERR_DEVICE, "device allocation for the model failed"));
   if (upload_pageable(m->d_ham, ham, sizeof(double) * 2 * n2 * n_R) != RTB_OK) return cleanup(RTB_ERR_DEVICE);
-  if (hipMemcpy(m->d_R, R.data(), sizeof(double) * R.size(), hipMemcpyHostToDevice) != hipSuccess ||
+  if (hipMemcpy(m->d_pairs, pairs.data(), sizeof(int) * pairs.size(), hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemcpy(m->d_R, R.data(), sizeof(double) * R.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(m->d_Rcart, Rc.data(), sizeof(double) * Rc.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(m->d_tau, tau.data(), sizeof(double) * tau.size(), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(m->d_taucart, tauc.data(), sizeof(double) * tauc.size(), hipMemcpyHostToDevice) != hipSuccess)
@@ -718,6 +748,7 @@ int rtb_model_create(int dim, int spin, int norb, int n_R, const int64_t* hamR, 
 void rtb_model_destroy(rtb_model* m) {
   if (!m) return;
   (void)hipFree(m->d_ham);
+  (void)hipFree(m->d_pairs);
   (void)hipFree(m->d_R);
   (void)hipFree(m->d_Rcart);
   (void)hipFree(m->d_tau);

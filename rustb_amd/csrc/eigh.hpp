@@ -93,6 +93,8 @@ struct FourierArgs {
   const double* wR;       // [np][nR]  w_p . R_cart
   const double* tau;      // [n][3]    fractional
   const double* wtau;     // [np][n]   w_p . tau_cart
+  int npair = 0;              // every stored R once, with -R where that is stored:
+  const int* pairs = nullptr;  // [npair] (r, index of -R or -1)
 };
 // k: [nk][3] (zero padded); H: [nk][n][n]; V: [nk][np][n][n] (or null when
 // np == 0; [nk][n][n] with a.combine)

@@ -1,13 +1,11 @@
 // Bloch Fourier sum H(k) = sum_R e^{i 2 pi k.R} h_R and its projected
 // k-derivatives (model_physics.rs:43-148, velocity.rs:470-731), FP64.
 //
-// Dense form: for a tile of TK k-points, every thread owns one matrix element
-// e = (m, c) and accumulates, in stored R order, U_R h_R[e] for H and
-// (w_p . R_cart) U_R h_R[e] for each projected direction p.  The phase table
-// U[kk][r] of the tile is generated in LDS with the k.R argument reduced mod 1
-// in FP64 before sincospi.  h_R[e] is read once per R and reused by the TK
-// k-points of the tile (coalesced along e).  Epilogue: the Atom-gauge
-// similarity conj(phi_m) phi_c and the tau term i (w.tau_c - w.tau_m) H_lat.
+// Dense form: a product on the matrix cores of the phases of a tile of k-points,
+// generated in LDS with the k.R argument reduced mod 1 in FP64 before sincospi,
+// and the hoppings of a tile of elements e = (m, c), over pairs R, -R.
+// Epilogue: the Atom-gauge similarity conj(phi_m) phi_c and the tau term
+// i (w.tau_c - w.tau_m) H_lat.
 #include <algorithm>
 
 #include "eigh.hpp"
@@ -18,6 +16,7 @@ namespace {
 
 constexpr int kRC = 32;     // R values staged per LDS round
 constexpr int kBlock = 256; // threads per workgroup
+constexpr int kDies = 8;    // XCDs, dealt workgroups in turn
 
 __device__ inline void phase_of(double arg, double& c, double& s) {
   // exp(i 2 pi arg), arg reduced to [-1/2, 1/2] first
@@ -25,27 +24,24 @@ __device__ inline void phase_of(double arg, double& c, double& s) {
   sincospi(2.0 * t, &s, &c);
 }
 
-// The epilogue of one k-point kv and element e = (m, c) of its matrices:
-// the Atom-gauge factor conj(phi_m) phi_c, the tau term of the projected
-// velocities, the stores.  ho: complex index of element e of H(k); vo: of
+// exp(i 2 pi k.tau) of orbital o
+__device__ inline double2 orbital_phase(const FourierArgs& a, const double* kv, int o) {
+  const double* t = a.tau + static_cast<size_t>(o) * 3;
+  double2 u;
+  phase_of(t[0] * kv[0] + t[1] * kv[1] + t[2] * kv[2], u.x, u.y);
+  return u;
+}
+
+// The epilogue of one k-point and element e = (m, c) of its matrices: the
+// Atom-gauge factor g = conj(phi_m) phi_c, each phase as in the reference, the
+// tau term of the projected velocities, the stores.  ho: complex index of
+// element e of H(k); vo: of
 // element e of the first V matrix of k (NP matrices per k, or one holding
 // V0 + i V1 with a.combine).
 template <int NP>
-__device__ inline void store_elem(const FourierArgs& a, const double* kv, int m, int c, double hr, double hi,
+__device__ inline void store_elem(const FourierArgs& a, double gr, double gi, int m, int c, double hr, double hi,
                                   const double* vr, const double* vi, double* __restrict__ H, size_t ho,
                                   double* __restrict__ V, size_t vo, size_t n2) {
-  double gr = 1.0, gi = 0.0;
-  if (a.gauge == RTB_GAUGE_ATOM) {
-    // conj(phi_m) phi_c = exp(i 2 pi k.(tau_c - tau_m)); each phase as in the
-    // reference, exp(i 2 pi k.tau) per orbital, multiplied
-    const double* tm = a.tau + static_cast<size_t>(m) * 3;
-    const double* tc = a.tau + static_cast<size_t>(c) * 3;
-    double cm, sm, cc, sc;
-    phase_of(tm[0] * kv[0] + tm[1] * kv[1] + tm[2] * kv[2], cm, sm);
-    phase_of(tc[0] * kv[0] + tc[1] * kv[1] + tc[2] * kv[2], cc, sc);
-    gr = cm * cc + sm * sc;
-    gi = cm * sc - sm * cc;
-  }
   H[2 * ho] = hr * gr - hi * gi;
   H[2 * ho + 1] = hr * gi + hi * gr;
   double cr = 0.0, ci = 0.0;
@@ -76,101 +72,156 @@ __device__ inline void store_elem(const FourierArgs& a, const double* kv, int m,
   }
 }
 
-template <int TK, int NP>
-__global__ void __launch_bounds__(kBlock) fourier_dense_kernel(FourierArgs a, const double* __restrict__ k,
-                                                               int nk, double* __restrict__ H,
-                                                               double* __restrict__ V) {
-  __shared__ double Ur[TK][kRC];
-  __shared__ double Ui[TK][kRC];
-  __shared__ double W[NP > 0 ? NP : 1][kRC];
-  __shared__ double Ks[TK][3];
+// ---- the sum over pairs (R, -R) on the FP64 matrix cores ----
+//
+// U_-R = conj(U_R) and w.(-R) = -w.R, so with E = h_R + h_-R, O = h_R - h_-R
+// (h_-R = 0 where -R is not stored) and U_R = c + i s a pair adds
+//   H: (c Ex - s Oy) + i (c Ey + s Ox),   V: w ((c Ox - s Ey) + i (c Oy + s Ex)),
+// 6 multiply-adds per stored R for H and two velocities where the sum over
+// single R takes 10 instructions, and a product of k-points by pairs with
+// pairs by elements: v_mfma_f64_16x16x4 with the k-points as rows (c, s and
+// w c, w s from LDS), 16 elements as columns, 4 pairs per instruction.  A wave
+// holds KT tiles of 16 k-points of 16 elements; its lane forms E and O of one
+// pair and element from two loads, issued a step ahead.  Workgroups are dealt
+// to the dies so that the k-tiles of one element tile meet in one L2.
+// Bound: the matrix cores (72 TFLOP/s), then the phases; n = 50, 343 R, 2431
+// k-points, H and two velocities 1078 -> 548 us (the products alone 350) against
+// the sum over single R on the vector units; n = 8, 125 R, 8 k-points, where the
+// chain of loads counted, 57 -> 17 us.
+constexpr int kPairChunk = 32;  // pairs whose phases are in LDS at a time
+constexpr int kPairElems = 64;  // elements per workgroup, 16 per wave
+
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+__device__ inline d4 mfma64(double a, double b, d4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+
+template <int NP, int KT>
+__global__ void __launch_bounds__(kBlock, NP == 3 && KT == 2 ? 2 : 3) fourier_dense_kernel(FourierArgs a, const double* __restrict__ k, int nk,
+                                                              int ktiles, int tiles, double* __restrict__ H,
+                                                              double* __restrict__ V) {
+  constexpr int KB = 16 * KT;  // k-points per workgroup
+  constexpr int ND = NP > 0 ? NP : 1;
+  __shared__ double2 U[kPairChunk * KB];  // [pair][k]; at the end [row m][k], at most 9 rows
+  __shared__ double W[kPairChunk][ND];
+  __shared__ double Ks[KB][3];
+  const int tile = static_cast<int>(blockIdx.x % kDies * (gridDim.x / kDies) + blockIdx.x / kDies);
+  if (tile >= tiles) return;
   const int n2 = a.n * a.n;
-  const int e = blockIdx.x * kBlock + threadIdx.x;
-  const int k0 = blockIdx.y * TK;
-  if (threadIdx.x < TK * 3) {
-    int kk = threadIdx.x / 3, d = threadIdx.x % 3;
-    Ks[kk][d] = (k0 + kk < nk) ? k[static_cast<size_t>(k0 + kk) * 3 + d] : 0.0;
-  }
-  double hr[TK], hi[TK];
-  double vr[NP > 0 ? NP : 1][TK], vi[NP > 0 ? NP : 1][TK];
+  const int k0 = tile % ktiles * KB;
+  const int lane = threadIdx.x % 64, fk = lane / 16;
+  const int e0 = tile / ktiles * kPairElems, e = e0 + threadIdx.x / 64 * 16 + lane % 16;
+  const int ec = min(e, n2 - 1);
+  for (int q = threadIdx.x; q < KB * 3; q += kBlock)
+    Ks[q / 3][q % 3] = k0 + q / 3 < nk ? k[static_cast<size_t>(k0) * 3 + q] : 0.0;
+  d4 hr[KT], hi[KT], vr[ND][KT], vi[ND][KT];
 #pragma unroll
-  for (int kk = 0; kk < TK; ++kk) {
-    hr[kk] = 0.0;
-    hi[kk] = 0.0;
+  for (int t = 0; t < KT; ++t) {
+    hr[t] = hi[t] = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      vr[p][kk] = 0.0;
-      vi[p][kk] = 0.0;
-    }
+    for (int p = 0; p < ND; ++p) vr[p][t] = vi[p][t] = d4{0.0, 0.0, 0.0, 0.0};
   }
   const double2* ham2 = reinterpret_cast<const double2*>(a.ham);
-  for (int R0 = 0; R0 < a.nR; R0 += kRC) {
-    __syncthreads();
-    const int rc = min(kRC, a.nR - R0);
-    for (int q = threadIdx.x; q < TK * kRC; q += kBlock) {
-      int kk = q / kRC, r = q % kRC;
-      double c = 0.0, s = 0.0;
-      if (r < rc && k0 + kk < nk) {
-        const double* Rv = a.R + static_cast<size_t>(R0 + r) * 3;
-        // same association as the reference: R0*k0 + R1*k1 + R2*k2
-        double arg = Rv[0] * Ks[kk][0] + Rv[1] * Ks[kk][1] + Rv[2] * Ks[kk][2];
-        phase_of(arg, c, s);
-      }
-      Ur[kk][r] = c;
-      Ui[kk][r] = s;
-    }
-    for (int q = threadIdx.x; q < NP * kRC; q += kBlock) {
-      int p = q / kRC, r = q % kRC;
-      W[p][r] = r < rc ? a.wR[static_cast<size_t>(p) * a.nR + R0 + r] : 0.0;
-    }
-    __syncthreads();
-    if (e < n2) {
-      for (int r = 0; r < rc; ++r) {
-        const double2 h = ham2[static_cast<size_t>(R0 + r) * n2 + e];
-#pragma unroll
-        for (int kk = 0; kk < TK; ++kk) {
-          const double ur = Ur[kk][r], ui = Ui[kk][r];
-          const double tr = ur * h.x - ui * h.y;
-          const double ti = ur * h.y + ui * h.x;
-          hr[kk] += tr;
-          hi[kk] += ti;
-#pragma unroll
-          for (int p = 0; p < NP; ++p) {
-            vr[p][kk] += W[p][r] * tr;
-            vi[p][kk] += W[p][r] * ti;
-          }
+  const int2* pairs = reinterpret_cast<const int2*>(a.pairs);
+  const int steps = (a.npair + 3) / 4;
+  auto entry = [&](int s) { return pairs[min(4 * s + fk, a.npair - 1)]; };  // the last repeats, with phase 0
+  auto load = [&](int r) { return ham2[static_cast<size_t>(r) * n2 + ec]; };
+  int2 now = entry(0), nxt = entry(1);
+  double2 x = load(now.x), y = load(max(now.y, 0));
+  for (int s = 0; s < steps; ++s) {
+    const int c0 = s / (kPairChunk / 4) * kPairChunk;
+    if (4 * s == c0) {
+      __syncthreads();
+      for (int q = threadIdx.x; q < KB * kPairChunk; q += kBlock) {
+        const int kk = q % KB, p = q / KB;
+        double c = 0.0, si = 0.0;
+        if (c0 + p < a.npair && k0 + kk < nk) {
+          const double* Rv = a.R + static_cast<size_t>(pairs[c0 + p].x) * 3;
+          // same association as the reference: R0*k0 + R1*k1 + R2*k2
+          const double arg = Rv[0] * Ks[kk][0] + Rv[1] * Ks[kk][1] + Rv[2] * Ks[kk][2];
+          phase_of(arg, c, si);
         }
+        U[q] = make_double2(c, si);
+      }
+      for (int q = threadIdx.x; q < NP * kPairChunk; q += kBlock) {
+        const int d = q % ND, p = q / ND;
+        W[p][d] = c0 + p < a.npair ? a.wR[static_cast<size_t>(d) * a.nR + pairs[c0 + p].x] : 0.0;
+      }
+      __syncthreads();
+    }
+    const double f = now.y >= 0 ? 1.0 : 0.0;
+    const double ex = fma(f, y.x, x.x), ey = fma(f, y.y, x.y), ox = fma(-f, y.x, x.x), oy = fma(-f, y.y, x.y);
+    now = nxt;
+    x = load(now.x);
+    y = load(max(now.y, 0));
+    nxt = entry(s + 2);
+    const int p = 4 * s - c0 + fk;
+    double w[ND];
+#pragma unroll
+    for (int d = 0; d < NP; ++d) w[d] = W[p][d];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+      const double2 u = U[p * KB + 16 * t + lane % 16];
+      hr[t] = mfma64(u.x, ex, hr[t]);
+      hi[t] = mfma64(u.x, ey, hi[t]);
+      hr[t] = mfma64(u.y, -oy, hr[t]);
+      hi[t] = mfma64(u.y, ox, hi[t]);
+#pragma unroll
+      for (int d = 0; d < NP; ++d) {
+        const double wc = w[d] * u.x, ws = w[d] * u.y;
+        vr[d][t] = mfma64(wc, ox, vr[d][t]);
+        vi[d][t] = mfma64(wc, oy, vi[d][t]);
+        vr[d][t] = mfma64(ws, -ey, vr[d][t]);
+        vi[d][t] = mfma64(ws, ex, vi[d][t]);
       }
     }
+  }
+  // phases of the rows m the workgroup's elements lie in; a lane's column c
+  // is its own
+  const bool atom = a.gauge == RTB_GAUGE_ATOM;
+  const int m0 = e0 / a.n, m1 = (min(e0 + kPairElems, n2) - 1) / a.n;
+  if (atom) {
+    __syncthreads();
+    for (int q = threadIdx.x; q < (m1 - m0 + 1) * KB; q += kBlock) U[q] = orbital_phase(a, Ks[q % KB], m0 + q / KB);
+    __syncthreads();
   }
   if (e >= n2) return;
   const int m = e / a.n, c = e % a.n;
 #pragma unroll
-  for (int kk = 0; kk < TK; ++kk) {
-    const int kg = k0 + kk;
-    if (kg >= nk) break;
-    double pr[NP > 0 ? NP : 1], pi[NP > 0 ? NP : 1];
+  for (int t = 0; t < KT; ++t)
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
-      pr[p] = vr[p][kk];
-      pi[p] = vi[p][kk];
+    for (int r = 0; r < 4; ++r) {
+      const int kk = 16 * t + 4 * r + fk;
+      const int kg = k0 + kk;
+      if (kg >= nk) continue;
+      double pr[ND], pi[ND];
+#pragma unroll
+      for (int p = 0; p < NP; ++p) {
+        pr[p] = vr[p][t][r];
+        pi[p] = vi[p][t][r];
+      }
+      const size_t ho = static_cast<size_t>(kg) * n2 + e;
+      const size_t vo = static_cast<size_t>(kg) * (NP == 2 && a.combine ? 1 : NP) * n2 + e;
+      double gr = 1.0, gi = 0.0;
+      if (atom) {
+        const double2 um = U[(m - m0) * KB + kk], uc = orbital_phase(a, Ks[kk], c);
+        gr = um.x * uc.x + um.y * uc.y;
+        gi = um.x * uc.y - um.y * uc.x;
+      }
+      store_elem<NP>(a, gr, gi, m, c, hr[t][r], hi[t][r], pr, pi, H, ho, V, vo, n2);
     }
-    const size_t ho = static_cast<size_t>(kg) * n2 + e;
-    const size_t vo = static_cast<size_t>(kg) * (NP == 2 && a.combine ? 1 : NP) * n2 + e;
-    store_elem<NP>(a, Ks[kk], m, c, hr[kk], hi[kk], pr, pi, H, ho, V, vo, n2);
-  }
 }
 
-template <int TK, int NP>
-int launch_dense(hipStream_t st, const FourierArgs& a, const double* k, size_t nk, double* H, double* V) {
-  const int n2 = a.n * a.n;
-  const size_t maxy = 65535;
-  for (size_t off = 0; off < nk; off += maxy * TK) {
-    size_t cnt = nk - off < maxy * TK ? nk - off : maxy * TK;
-    dim3 grid((n2 + kBlock - 1) / kBlock, static_cast<unsigned>((cnt + TK - 1) / TK));
-    hipLaunchKernelGGL((fourier_dense_kernel<TK, NP>), grid, dim3(kBlock), 0, st, a, k + off * 3,
-                       static_cast<int>(cnt), H + off * static_cast<size_t>(n2) * 2,
-                       V ? V + off * static_cast<size_t>(NP) * n2 * 2 : nullptr);
+template <int NP, int KT>
+int launch_tiles(hipStream_t st, const FourierArgs& a, const double* k, size_t nk, double* H, double* V) {
+  const size_t n2 = static_cast<size_t>(a.n) * a.n, etiles = (n2 + kPairElems - 1) / kPairElems;
+  const size_t maxk = (size_t(1) << 30) / etiles / (16 * KT) * (16 * KT);  // tiles of a launch within an int
+  const size_t vk = NP == 2 && a.combine ? 1 : NP;
+  for (size_t off = 0; off < nk; off += maxk) {
+    const size_t cnt = std::min(nk - off, maxk), ktiles = (cnt + 16 * KT - 1) / (16 * KT);
+    const size_t tiles = ktiles * etiles, grid = (tiles + kDies - 1) / kDies * kDies;
+    hipLaunchKernelGGL((fourier_dense_kernel<NP, KT>), dim3(static_cast<unsigned>(grid)), dim3(kBlock), 0, st, a,
+                       k + off * 3, static_cast<int>(cnt), static_cast<int>(ktiles), static_cast<int>(tiles),
+                       H + off * n2 * 2, V ? V + off * vk * n2 * 2 : nullptr);
   }
   RTB_HIP(hipGetLastError());
   return RTB_OK;
@@ -186,8 +237,8 @@ int launch_dense(hipStream_t st, const FourierArgs& a, const double* k, size_t n
 // G = 1 and the tile is one 256-element block.  Workgroups take tile indices from
 // one atomic counter in the order of the table (the host sorts it by cost,
 // longest first) until the table is exhausted, so every workgroup exits once
-// the counter passes the tile count.  Per (R, element, k) the arithmetic is
-// the dense kernel's: the same phases, stored R order and epilogue.
+// the counter passes the tile count.  Per (R, element, k) the phases
+// and the epilogue are the dense kernel's; the sum runs in stored R order.
 template <int TK>
 __global__ void __launch_bounds__(kBlock) fourier_queue_kernel(const QueueModel* __restrict__ models,
                                                                const QueueTile* __restrict__ tiles, int ntiles,
@@ -283,7 +334,13 @@ __global__ void __launch_bounds__(kBlock) fourier_queue_kernel(const QueueModel*
       const int kq = grp * TK + kk;
       if (kq >= kn) break;
       const double pr[2] = {vr[0][kk], vr[1][kk]}, pi[2] = {vi[0][kk], vi[1][kk]};
-      store_elem<2>(a, Ks[kq], m, c, hr[kk], hi[kk], pr, pi, tile.H, static_cast<size_t>(kq) * n2 + e, tile.V,
+      double gr = 1.0, gi = 0.0;
+      if (a.gauge == RTB_GAUGE_ATOM) {
+        const double2 um = orbital_phase(a, Ks[kq], m), uc = orbital_phase(a, Ks[kq], c);
+        gr = um.x * uc.x + um.y * uc.y;
+        gi = um.x * uc.y - um.y * uc.x;
+      }
+      store_elem<2>(a, gr, gi, m, c, hr[kk], hi[kk], pr, pi, tile.H, static_cast<size_t>(kq) * n2 + e, tile.V,
                     static_cast<size_t>(kq) * vper * n2 + e, static_cast<size_t>(n2));
     }
   }
@@ -314,19 +371,30 @@ __global__ void mesh_points_kernel(int dim, unsigned long long n1, unsigned long
   o[2] = dim >= 3 ? static_cast<double>(i3) / static_cast<double>(n3) : 0.0;
 }
 
+// Two k-tiles per wave share the loads and E, O where that still gives every CU
+// two workgroups; below, the CUs left idle cost more (n = 18, 301 k-points: 231
+// workgroups of two tiles, 399 of one).
+template <int NP>
+int launch_dense(hipStream_t st, const FourierArgs& a, const double* k, size_t nk, double* H, double* V) {
+  const size_t etiles = (static_cast<size_t>(a.n) * a.n + kPairElems - 1) / kPairElems;
+  return etiles * ((nk + 31) / 32) >= 512 ? launch_tiles<NP, 2>(st, a, k, nk, H, V)
+                                          : launch_tiles<NP, 1>(st, a, k, nk, H, V);
+}
+
 }  // namespace
 
 int fourier_dense(hipStream_t st, const FourierArgs& a, const double* k, size_t nk, double* H, double* V) {
   if (nk == 0) return RTB_OK;
+  if (a.npair < 1) return fail(RTB_ERR_INVALID_MODEL, "a model holds no hoppings");
   switch (a.np) {
     case 0:
-      return launch_dense<8, 0>(st, a, k, nk, H, nullptr);
+      return launch_dense<0>(st, a, k, nk, H, nullptr);
     case 1:
-      return launch_dense<8, 1>(st, a, k, nk, H, V);
+      return launch_dense<1>(st, a, k, nk, H, V);
     case 2:
-      return launch_dense<8, 2>(st, a, k, nk, H, V);
+      return launch_dense<2>(st, a, k, nk, H, V);
     case 3:
-      return launch_dense<8, 3>(st, a, k, nk, H, V);
+      return launch_dense<3>(st, a, k, nk, H, V);
     default:
       return fail(RTB_ERR_UNSUPPORTED, "at most 3 projected directions");
   }

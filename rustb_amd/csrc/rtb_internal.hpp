@@ -258,6 +258,8 @@ struct rtb_model {
   double* d_ham = nullptr;    // [nR][n][n] complex (re, im)
   double* d_R = nullptr;      // [nR][3]   R as doubles (zero padded)
   double* d_Rcart = nullptr;  // [nR][3]   R . lat
+  int npair = 0;
+  int* d_pairs = nullptr;     // [npair] (r, index of -R or -1): every stored R once
   double* d_tau = nullptr;    // [n][3]    fractional tau, spin duplicated
   double* d_taucart = nullptr;  // [n][3]  tau . lat
 };
