@@ -489,27 +489,32 @@ __global__ void __launch_bounds__(256) cut_mu_kernel(cut::View V, const double* 
 // order and divided by their count into M, as the host walk forms them;
 // then greedy_assign (tracking.rs:44-68): rows by descending row maximum
 // (stable), each taking its largest unassigned column, the lowest column
-// among equal values.  A row whose overall best column (same scan rule) is
-// still free takes it, which is what the scan over the free columns returns;
-// otherwise wave 0 scans the free columns.  The same operations on the same
-// values as the host walk, so the permutations are identical.  M [n][n] sits
-// in LDS up to kTrackLdsMaxN bands and above in a global slice per
-// workgroup of the launch (n = 256: 512 KiB); there a wave builds each row
-// and ranks its first kTrackTop columns in registers, a row whose best
-// column is taken takes the first free one of them, and only when all are
-// taken does wave 0 scan the row in global memory.
+// among equal values.  Where all rows' best columns differ each row takes its
+// own; otherwise the rows are ranked and wave 0 walks only those whose best
+// column is taken when their turn comes, each scanning the free columns.  The
+// same operations on the same values as the host walk, so the permutations
+// are identical.  M [n][n] sits in LDS up to kTrackLdsMaxN bands and above in
+// a global slice per workgroup of the launch (n = 256: 512 KiB); there a wave
+// builds each row and ranks its first kTrackTop columns in registers, a row
+// whose best column is taken takes the first free one of them, and only when
+// all are taken does wave 0 scan the row in global memory.
+// Bound: a chain of launches, one per level (4.3 us each where they do next to
+// nothing, n = 4); in one, the latencies of schedule, permutations and overlaps
+// in turn.  Per level, 2D: n = 32 14.8 -> 7.7 us, n = 64 32 -> 15, n = 128
+// 89 -> 43, n = 160 136 -> 101 against a thread per row's maximum and a walk of
+// every row.
 constexpr int kTrackMaxDep = 6;  // visited neighbours of a 3D vertex at most
 static_assert(sizeof(TrackEntry) == 8 * sizeof(unsigned), "schedule entry layout");
 static_assert(kTrackDevMaxN <= 256, "the greedy's assigned-column mask is four 64-bit words");
 
-// LDS bytes: M when it is in LDS, then rmax [n], best/order/bsort [n] each,
+// LDS bytes: M when it is in LDS, then rmax [n], best/order/bsort/owner [n] each,
 // the neighbours' permutations [kTrackMaxDep][n] and, with M in global
 // memory, each row's first kTrackTop columns [n][kTrackTop]
 constexpr int kTrackTop = 4;
 size_t track_smem(int n) {
   const bool lds = n <= kTrackLdsMaxN;
   const size_t m = lds ? static_cast<size_t>(n) * n * sizeof(double) : 0;
-  return m + n * sizeof(double) + (3 + kTrackMaxDep + (lds ? 0 : kTrackTop)) * static_cast<size_t>(n) * sizeof(int);
+  return m + n * sizeof(double) + (4 + kTrackMaxDep + (lds ? 0 : kTrackTop)) * static_cast<size_t>(n) * sizeof(int);
 }
 
 __global__ void identity_perm_kernel(size_t total, int n, int* __restrict__ perm) {
@@ -524,11 +529,11 @@ __device__ inline double by_count(double x, int cnt, double dc) {
   return cnt == 1 ? x : (cnt == 2 ? x * 0.5 : (cnt == 4 ? x * 0.25 : x / dc));
 }
 
-// kTrackThreads per vertex with M in LDS (one wave of 64 was slower at
-// n = 32: the matrix build loses its parallelism); with M in global memory
-// kTrackThreadsWide, one row per wave in flight: the build waits on global
-// loads, and a level holds few vertices.
-constexpr int kTrackThreads = 256;
+// Threads per vertex: the build waits on loads, and a level holds few vertices,
+// so as many rows at once as fit (n = 32, 128 x 128: 3.63 ms with 256 threads,
+// 2.95 with 512, 2.63 with 1024; n <= 16 the same within 4%); with M in global
+// memory one row per wave in flight.
+constexpr int kTrackThreads = 1024;
 constexpr int kTrackThreadsWide = 1024;
 template <bool kLdsM>
 __global__ void __launch_bounds__(kLdsM ? kTrackThreads : kTrackThreadsWide) track_kernel(const double* __restrict__ ovx, const double* __restrict__ ovy,
@@ -544,13 +549,17 @@ __global__ void __launch_bounds__(kLdsM ? kTrackThreads : kTrackThreadsWide) tra
   int* best = reinterpret_cast<int*>(rmax + n);          // [n] each row's best column over all columns
   int* order = best + n;                                 // [n] rows by descending maximum
   int* bsort = order + n;                                // [n] best[order[s]]
-  int* pv = bsort + n;                                   // [kTrackMaxDep][n] the neighbours' permutations
+  int* owner = bsort + n;                                // [n] a column's first rank
+  int* pv = owner + n;                                   // [kTrackMaxDep][n] the neighbours' permutations
   int* top = pv + kTrackMaxDep * n;                      // [n][kTrackTop] (M in global memory only)
   const TrackEntry te = sched[blockIdx.x];              // uniform: one scalar load
   const size_t nb = te.v;
   const int cnt = static_cast<int>(te.cnt);
   if (cnt == 0) return;  // vertex 0 keeps the identity
   const int tid = threadIdx.x;
+  __shared__ unsigned long long claimed[kTrackDevMaxN / 64];  // columns that are some row's best
+  if (tid < kTrackDevMaxN / 64) claimed[tid] = 0;
+  for (int a = tid; a < n; a += NT) owner[a] = n;
 #pragma unroll
   for (int r = 0; r < kTrackMaxDep; ++r)
     if (r < cnt)
@@ -588,27 +597,34 @@ __global__ void __launch_bounds__(kLdsM ? kTrackThreads : kTrackThreadsWide) tra
     return by_count(x, cnt, dc);
   };
   if constexpr (kLdsM) {
-    for (int e = tid; e < nn; e += NT) {
-      const int a = e / n;
-      M[e] = entry(a, e - a * n);
-    }
-    __syncthreads();
-    // each row's maximum (fmax from -1: NaN dropped) and best column, the
-    // lowest among equal values: a row per thread, the scan rotated to
-    // spread the LDS banks
-    for (int i = tid; i < n; i += NT) {
+    // a row per group of sw lanes (16, 32 or a wave, the least that holds it
+    // or 64): built, stored and its maximum (NaN never ranked) and best
+    // column, the lowest among equal values, merged over the group
+    const int sw = n <= 16 ? 16 : (n <= 32 ? 32 : 64);
+    for (int a = tid / sw; a < n; a += NT / sw) {
       double bv = -1.0;
       int bj = 0;
-      for (int q = 0; q < n; ++q) {
-        const int j = q + i < n ? q + i : q + i - n;
-        const double v = M[i * n + j];
-        if (v > bv || (v == bv && j < bj)) {
-          bv = v;
-          bj = j;
+      for (int b = tid % sw; b < n; b += sw) {
+        const double x = entry(a, b);
+        M[a * n + b] = x;
+        if (x > bv) {
+          bv = x;
+          bj = b;
         }
       }
-      rmax[i] = bv;
-      best[i] = bj;
+      for (int o = sw / 2; o > 0; o >>= 1) {
+        const double ov = __shfl_xor(bv, o);
+        const int oj = __shfl_xor(bj, o);
+        if (ov > bv || (ov == bv && oj < bj)) {
+          bv = ov;
+          bj = oj;
+        }
+      }
+      if (tid % sw == 0) {
+        rmax[a] = bv;
+        best[a] = bj;
+        atomicOr(&claimed[bj >> 6], 1ull << (bj & 63));
+      }
     }
   } else {
     // a row per wave, each lane its columns b = lane + 64 c: the row is
@@ -659,6 +675,7 @@ __global__ void __launch_bounds__(kLdsM ? kTrackThreads : kTrackThreadsWide) tra
           if (k == 0) {
             rmax[a] = bv;
             best[a] = bj;
+            atomicOr(&claimed[bj >> 6], 1ull << (bj & 63));
           }
           top[a * kTrackTop + k] = bv >= 0.0 ? bj : -1;  // -1: no further candidate
         }
@@ -668,98 +685,111 @@ __global__ void __launch_bounds__(kLdsM ? kTrackThreads : kTrackThreadsWide) tra
     }
   }
   __syncthreads();
-  // the stable descending sort as ranks
+  int* out = perm + nb * n;
+  // where no column is the best of two rows each row takes its own, whatever
+  // the order
+  int distinct = 0;
+  for (int c = 0; c < kTrackDevMaxN / 64; ++c) distinct += __popcll(claimed[c]);
+  if (distinct == n) {
+    for (int i = tid; i < n; i += NT) out[i] = best[i];
+    return;
+  }
+  // the stable descending sort as ranks; owner: the first rank a column is
+  // the best of
   for (int i = tid; i < n; i += NT) {
     const double x = rmax[i];
     int rank = 0;
+#pragma unroll 8
     for (int k = 0; k < n; ++k) {
       const double y = rmax[k];
       rank += (y > x || (y == x && k < i)) ? 1 : 0;
     }
     order[rank] = i;
     bsort[rank] = best[i];
+    atomicMin(&owner[best[i]], rank);
   }
   __syncthreads();
   if (tid >= 64) return;
   const int lane = tid;
-  // assigned columns 64 c .. 64 c + 63 in word c (the same in every lane);
-  // NW named words rather than an array indexed at run time
+  // Ranks that do not get their best column, 64 c .. 64 c + 63 in word c (the
+  // same in every lane): those whose column has an earlier owner and, as the
+  // walk finds them, those whose column a displaced row before them takes.
+  // At rank s a column is taken if its owner comes before s (the owner has it
+  // or found it taken) or a displaced row took it; bits: the latter's columns.
   constexpr int NW = kLdsM ? kTrackLdsMaxN / 64 : kTrackDevMaxN / 64;
-  static_assert(NW == 2 || NW == 4, "two or four assigned-column words");
-  unsigned long long tk0 = 0, tk1 = 0, tk2 = 0, tk3 = 0;
-  const auto word = [&](int c) {
-    if constexpr (NW == 2) return c == 0 ? tk0 : tk1;
-    return c == 0 ? tk0 : (c == 1 ? tk1 : (c == 2 ? tk2 : tk3));
-  };
-  const auto taken = [&](int j) { return ((word(j >> 6) >> (j & 63)) & 1ull) != 0; };
-  int* out = perm + nb * n;
-  int r_next = order[0], j_next = bsort[0];  // read one step ahead
-  for (int s = 0; s < n; ++s) {
-    const int r = r_next;
-    int j = j_next;
-    if (s + 1 < n) {
-      r_next = order[s + 1];
-      j_next = bsort[s + 1];
-    }
-    bool scan = taken(j);  // the same in every lane
-    if constexpr (!kLdsM) {
-      // the first free column of the row's ranked list (entry 0 is j) is the
-      // free columns' maximum; the full scan only when the list runs out
-      if (scan) {
+  unsigned long long late[NW], bits[NW];
+  int own[NW];  // of columns lane + 64 c
+#pragma unroll
+  for (int c = 0; c < NW; ++c) {
+    const int s = lane + 64 * c;
+    late[c] = __ballot(s < n && owner[s < n ? bsort[s] : 0] != s);
+    bits[c] = 0;
+    own[c] = s < n ? owner[s] : 0;
+  }
+#pragma unroll
+  for (int w = 0; w < NW; ++w) {
+    while (late[w]) {
+      const int q = __ffsll(late[w]) - 1, s = 64 * w + q;
+      late[w] &= late[w] - 1;
+      const int r = order[s];
+      int j = -1;
+      if constexpr (!kLdsM) {
+        // the first free column of the row's ranked list (entry 0 is its best)
+        // is the free columns' maximum; the full scan only when the list runs
+        // out
 #pragma unroll
         for (int k = 1; k < kTrackTop; ++k) {
           const int c = top[r * kTrackTop + k];
           if (c < 0) break;
-          if (!taken(c)) {
+          bool t = owner[c] < s;
+#pragma unroll
+          for (int v = 0; v < NW; ++v) t = t || (v == c >> 6 && ((bits[v] >> (c & 63)) & 1ull));
+          if (!t) {
             j = c;
-            scan = false;
             break;
           }
         }
       }
-    }
-    if (scan) {  // the scan over the free columns
-      // no candidate: (-1, 0), as the host scan's start; every real
-      // candidate is >= 0 and NaN never wins
-      double bv = -1.0;
-      int bj = 0;
+      if (j < 0) {  // the scan over the free columns
+        // no candidate: (-1, 0), as the host scan's start; every real
+        // candidate is >= 0 and NaN never wins
+        double bv = -1.0;
+        int bj = 0;
 #pragma unroll
-      for (int c = 0; c < NW; ++c) {
-        const int jj = lane + 64 * c;
-        if (jj < n) {
-          const bool t = (word(c) >> lane) & 1ull;
-          const double v = M[static_cast<size_t>(r) * n + jj];
-          if (!t && v > bv) {
-            bv = v;
-            bj = jj;
+        for (int c = 0; c < NW; ++c) {
+          const int jj = lane + 64 * c;
+          if (jj < n) {
+            const double v = M[static_cast<size_t>(r) * n + jj];
+            if (!(own[c] < s || ((bits[c] >> lane) & 1ull)) && v > bv) {
+              bv = v;
+              bj = jj;
+            }
           }
         }
-      }
-      for (int o = 32; o > 0; o >>= 1) {
-        const double ov = __shfl_xor(bv, o);
-        const int oj = __shfl_xor(bj, o);
-        if (ov > bv || (ov == bv && oj < bj)) {
-          bv = ov;
-          bj = oj;
+        for (int o = 32; o > 0; o >>= 1) {
+          const double ov = __shfl_xor(bv, o);
+          const int oj = __shfl_xor(bj, o);
+          if (ov > bv || (ov == bv && oj < bj)) {
+            bv = ov;
+            bj = oj;
+          }
         }
+        j = __builtin_amdgcn_readfirstlane(bj);
       }
-      j = bj;
-    }
-    const unsigned long long bit = 1ull << (j & 63);
-    if constexpr (NW == 2) {
-      if (j < 64)
-        tk0 |= bit;
-      else
-        tk1 |= bit;
-    } else {
-      switch (j >> 6) {
-        case 0: tk0 |= bit; break;
-        case 1: tk1 |= bit; break;
-        case 2: tk2 |= bit; break;
-        default: tk3 |= bit; break;
+      const int oj = owner[j];  // n: no row's best
+#pragma unroll
+      for (int c = 0; c < NW; ++c) {
+        if (j >> 6 == c) bits[c] |= 1ull << (j & 63);
+        if (oj > s && oj < n && oj >> 6 == c) late[c] |= 1ull << (oj & 63);
       }
+      if (lane == 0) bsort[s] = j;
     }
-    if (lane == 0) out[r] = j;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // bsort as lane 0 left it
+#pragma unroll
+  for (int c = 0; c < NW; ++c) {
+    const int s = lane + 64 * c;
+    if (s < n) out[order[s]] = bsort[s];
   }
 }
 

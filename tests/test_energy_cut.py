@@ -653,6 +653,19 @@ def test_gpu_device_walk_ragged_meshes(seed, mesh, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 31, 33, 63, 64, 65, 127, 129])
+def test_gpu_device_walk_at_group_edges(n, monkeypatch):
+    """The device walk equals the host walk bit for bit where the lanes per row
+    (16, 32, 64) and the words of the column masks (64 columns) change."""
+    m = wide_model(ra.Model, 50 + n, n, 2)
+    p = ra.Parameters.rank2((5, 4), [1.0, 0.0], [0.0, 1.0], np.linspace(-6, 6, 9), eta=0.05, integration="EnergyCut")
+    monkeypatch.delenv("RTB_TRACK_HOST", raising=False)
+    dev = m.hall_conductivity(p).conductivity
+    monkeypatch.setenv("RTB_TRACK_HOST", "1")
+    np.testing.assert_array_equal(dev, m.hall_conductivity(p).conductivity)
+
+
+@pytest.mark.gpu
 def test_gpu_n136_two_stage_vs_host_part():
     """n = 136: the vertex stage takes the two-stage FP64 eigensolver and the
     walk keeps each vertex's overlap matrix in a workspace slice; against the
