@@ -118,24 +118,28 @@ struct FinalArgs {
 };
 
 // Pass C for pairs [p0, p0 + gridDim.y): outputs in k1-innermost order.
-// A workgroup owns kTW matrix elements of one pair for all N1 values of k1:
-// the kTW columns of G0..G2 are staged in LDS once, and each thread forms
-// kFB values of k1 per pass, so one LDS read of G serves kFB outputs.  The
-// Atom-gauge factor conj(phi_m) phi_c = exp(i 2 pi (tau_c - tau_m).k) is one
-// sincospi per element and k.
-constexpr int kFB = 2;
+// A workgroup owns kTWF matrix elements of one pair for all N1 values of k1:
+// for each R1 = l it stages X = G0 and, the directions' weights being the same
+// for every k1, Q_p = alpha_p0 l G0 + alpha_p1 G1 + alpha_p2 G2 (with a.combine
+// Q_0 + i Q_1 alone), so that H and each velocity are one sum over l.  Each
+// thread forms kFB values of k1 per pass, so one LDS read serves kFB outputs.
+// The Atom-gauge factor conj(phi_m) phi_c = exp(i 2 pi (tau_c - tau_m).k) is
+// one sincospi per element and k.
+// Bound: the stores of H and V and the reads of G (n = 128, 48^3, 11 R1: 78 GB,
+// 16 ms at the copy rate): 27.5 -> 19.2 ms there, n = 32, 64^3, 5 R1 2.73 -> 2.11
+// ms against separate sums over G0, l G0, G1 and G2 (16 multiply-adds per l and
+// output, now 8) two values of k1 at a time.
+constexpr int kFB = 4;
 constexpr int kTWF = 64;  // matrix elements per workgroup of the final pass
 
-// NG: partial sums staged (G0 .. G_{NG-1}); VEL: the velocities are formed
-// (d1 from G0, then G1, G2 for NG = 2, 3).
-template <int NG, bool VEL>
+// NV: velocity matrices formed per k (0, 1 with a.combine, 2).
+template <int NV>
 __global__ void __launch_bounds__(256) dft_final_kernel(FinalArgs a, size_t p0, double2* __restrict__ H,
                                                         double2* __restrict__ V) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   double2* W = reinterpret_cast<double2*>(smem_raw);  // [N1]
-  double2* X0 = W + a.N1;                             // [L1][kTWF]
-  double2* X1 = X0 + a.L1 * kTWF;
-  double2* X2 = X1 + a.L1 * kTWF;
+  double2* X = W + a.N1;                              // [L1][1 + NV][kTWF]
+  constexpr int NX = 1 + NV, ND = NV > 0 ? NV : 1;
   const size_t n2 = static_cast<size_t>(a.n) * a.n;
   const size_t pl = blockIdx.y, pg = p0 + pl;
   const size_t t0 = static_cast<size_t>(blockIdx.x) * kTWF;
@@ -147,11 +151,26 @@ __global__ void __launch_bounds__(256) dft_final_kernel(FinalArgs a, size_t p0, 
   }
   for (int q = threadIdx.x; q < a.L1 * kTWF; q += 256) {
     const int l = q / kTWF, t = q % kTWF;
-    const size_t src = (static_cast<size_t>(l) * a.P + pg) * n2 + t0 + t;
-    const bool ok = t < tw;
-    X0[q] = ok ? a.G0[src] : make_double2(0.0, 0.0);
-    if (NG > 1) X1[q] = ok ? a.G1[src] : make_double2(0.0, 0.0);
-    if (NG > 2) X2[q] = ok ? a.G2[src] : make_double2(0.0, 0.0);
+    const size_t src = (static_cast<size_t>(l) * a.P + pg) * n2 + t0 + min(t, tw - 1);
+    const double2 x = a.G0[src];
+    double2* o = X + static_cast<size_t>(l) * NX * kTWF + t;
+    o[0] = x;
+    if (NV > 0) {
+      const double2 y = a.G1 ? a.G1[src] : make_double2(0.0, 0.0);
+      const double2 z = a.G2 ? a.G2[src] : make_double2(0.0, 0.0);
+      const double r1 = static_cast<double>(a.lo1 + l);
+      double2 v[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+        v[p] = make_double2(a.alpha[p][0] * (r1 * x.x) + a.alpha[p][1] * y.x + a.alpha[p][2] * z.x,
+                            a.alpha[p][0] * (r1 * x.y) + a.alpha[p][1] * y.y + a.alpha[p][2] * z.y);
+      if (NV == 1) {
+        o[kTWF] = make_double2(v[0].x - v[1].y, v[0].y + v[1].x);
+      } else {
+        o[kTWF] = v[0];
+        o[2 * kTWF] = v[1];
+      }
+    }
   }
   __syncthreads();
   const int t = threadIdx.x % kTWF;
@@ -169,24 +188,24 @@ __global__ void __launch_bounds__(256) dft_final_kernel(FinalArgs a, size_t p0, 
     wd[p] = a.wtau[static_cast<size_t>(p) * a.n + mcol] - a.wtau[static_cast<size_t>(p) * a.n + mrow];
   constexpr int kGroups = 256 / kTWF;
   for (int ib = (threadIdx.x / kTWF) * kFB; ib < a.N1; ib += kGroups * kFB) {
-    double hr[kFB], hi[kFB], d1r[kFB], d1i[kFB], g1r[kFB], g1i[kFB], g2r[kFB], g2i[kFB];
+    double hr[kFB], hi[kFB], vr[ND][kFB], vi[ND][kFB];
     int m[kFB], step[kFB];
 #pragma unroll
     for (int u = 0; u < kFB; ++u) {
       const int i1 = min(ib + u, a.N1 - 1);  // lanes past N1 repeat the last k1, unstored
       m[u] = dmod(i1 * a.lo1, a.N1);
       step[u] = i1;
-      hr[u] = hi[u] = d1r[u] = d1i[u] = g1r[u] = g1i[u] = g2r[u] = g2i[u] = 0.0;
+      hr[u] = hi[u] = 0.0;
+#pragma unroll
+      for (int p = 0; p < NV; ++p) vr[p][u] = vi[p][u] = 0.0;
     }
     // unrolled so that the LDS reads of the next terms are issued while the
     // current ones are multiplied
-#pragma unroll 4
+#pragma unroll 2
     for (int l = 0; l < a.L1; ++l) {
-      const double2 x = X0[l * kTWF + t];
-      const double2 y = NG > 1 ? X1[l * kTWF + t] : make_double2(0.0, 0.0);
-      const double2 z = NG > 2 ? X2[l * kTWF + t] : make_double2(0.0, 0.0);
-      const double r1 = static_cast<double>(a.lo1 + l);
-      double2 w[kFB];
+      double2 x[NX], w[kFB];
+#pragma unroll
+      for (int p = 0; p < NX; ++p) x[p] = X[(l * NX + p) * kTWF + t];
 #pragma unroll
       for (int u = 0; u < kFB; ++u) {
         w[u] = W[m[u]];
@@ -195,20 +214,12 @@ __global__ void __launch_bounds__(256) dft_final_kernel(FinalArgs a, size_t p0, 
       }
 #pragma unroll
       for (int u = 0; u < kFB; ++u) {
-        const double tr = w[u].x * x.x - w[u].y * x.y, ti = w[u].x * x.y + w[u].y * x.x;
-        hr[u] += tr;
-        hi[u] += ti;
-        if (VEL) {
-          d1r[u] += r1 * tr;
-          d1i[u] += r1 * ti;
-        }
-        if (NG > 1) {
-          g1r[u] += w[u].x * y.x - w[u].y * y.y;
-          g1i[u] += w[u].x * y.y + w[u].y * y.x;
-        }
-        if (NG > 2) {
-          g2r[u] += w[u].x * z.x - w[u].y * z.y;
-          g2i[u] += w[u].x * z.y + w[u].y * z.x;
+        hr[u] += w[u].x * x[0].x - w[u].y * x[0].y;
+        hi[u] += w[u].x * x[0].y + w[u].y * x[0].x;
+#pragma unroll
+        for (int p = 0; p < NV; ++p) {
+          vr[p][u] += w[u].x * x[1 + p].x - w[u].y * x[1 + p].y;
+          vi[p][u] += w[u].x * x[1 + p].y + w[u].y * x[1 + p].x;
         }
       }
     }
@@ -225,26 +236,23 @@ __global__ void __launch_bounds__(256) dft_final_kernel(FinalArgs a, size_t p0, 
       }
       const size_t kl = pl * a.N1 + i1;
       H[kl * n2 + e] = make_double2(hr[u] * gr - hi[u] * gi, hr[u] * gi + hi[u] * gr);
-      double cr = 0.0, ci = 0.0;
-      for (int p = 0; p < a.np; ++p) {
-        const double sr = a.alpha[p][0] * d1r[u] + a.alpha[p][1] * g1r[u] + a.alpha[p][2] * g2r[u];
-        const double si = a.alpha[p][0] * d1i[u] + a.alpha[p][1] * g1i[u] + a.alpha[p][2] * g2i[u];
-        double xr = -si, xi = sr;  // i * sum
+#pragma unroll
+      for (int p = 0; p < NV; ++p) {
+        double xr = -vi[p][u], xi = vr[p][u];  // i * sum
         if (a.gauge == RTB_GAUGE_ATOM) {
+          // + i (w_p . (tau_c - tau_m)) H, the directions combined as V is
           xr += -wd[p] * hi[u];
           xi += wd[p] * hr[u];
+          if (NV == 1) {
+            xr -= wd[1] * hr[u];
+            xi -= wd[1] * hi[u];
+          }
           const double yr = xr * gr - xi * gi, yi = xr * gi + xi * gr;
           xr = yr;
           xi = yi;
         }
-        if (a.combine) {
-          cr += p == 0 ? xr : -xi;
-          ci += p == 0 ? xi : xr;
-        } else {
-          V[(kl * 2 + p) * n2 + e] = make_double2(xr, xi);
-        }
+        V[(kl * NV + p) * n2 + e] = make_double2(xr, xi);
       }
-      if (a.combine && a.np == 2) V[kl * n2 + e] = make_double2(cr, ci);
     }
   }
 }
@@ -270,13 +278,11 @@ int mesh_set_smem_limits() {
   const int lim = 160 * 1024;
   RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dft_axis_kernel),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lim));
-  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dft_final_kernel<1, false>),
+  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dft_final_kernel<0>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lim));
-  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dft_final_kernel<1, true>),
+  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dft_final_kernel<1>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lim));
-  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dft_final_kernel<2, true>),
-                              hipFuncAttributeMaxDynamicSharedMemorySize, lim));
-  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dft_final_kernel<3, true>),
+  RTB_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&dft_final_kernel<2>),
                               hipFuncAttributeMaxDynamicSharedMemorySize, lim));
   return RTB_OK;
 }
@@ -397,23 +403,21 @@ int mesh_final(hipStream_t st, const rtb_model* m, const MeshPlan& p, const doub
   f.tau = a.tau;
   f.wtau = a.wtau;
   f.gauge = a.gauge;
-  const size_t smem = sizeof(double2) * (static_cast<size_t>(p.N[0]) + 3 * static_cast<size_t>(p.L[0]) * kTWF);
   const size_t tiles = (n2 + kTWF - 1) / kTWF;
   const size_t vk = f.combine ? 1 : 2;  // V matrices per k
+  const size_t smem =
+      sizeof(double2) * (static_cast<size_t>(p.N[0]) + (f.np ? 1 + vk : 1) * static_cast<size_t>(p.L[0]) * kTWF);
   for (size_t q0 = 0; q0 < np_pairs; q0 += 65535) {
     const size_t qc = np_pairs - q0 < 65535 ? np_pairs - q0 : 65535;
     const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>(qc));
     double2* Hq = reinterpret_cast<double2*>(H) + q0 * p.N[0] * n2;
     double2* Vq = V ? reinterpret_cast<double2*>(V) + q0 * p.N[0] * vk * n2 : nullptr;
-    if (!f.np) {
-      hipLaunchKernelGGL((dft_final_kernel<1, false>), grid, dim3(256), smem, st, f, p0 + q0, Hq, Vq);
-    } else if (f.dim == 1) {
-      hipLaunchKernelGGL((dft_final_kernel<1, true>), grid, dim3(256), smem, st, f, p0 + q0, Hq, Vq);
-    } else if (f.dim == 2) {
-      hipLaunchKernelGGL((dft_final_kernel<2, true>), grid, dim3(256), smem, st, f, p0 + q0, Hq, Vq);
-    } else {
-      hipLaunchKernelGGL((dft_final_kernel<3, true>), grid, dim3(256), smem, st, f, p0 + q0, Hq, Vq);
-    }
+    if (!f.np)
+      hipLaunchKernelGGL(dft_final_kernel<0>, grid, dim3(256), smem, st, f, p0 + q0, Hq, Vq);
+    else if (f.combine)
+      hipLaunchKernelGGL(dft_final_kernel<1>, grid, dim3(256), smem, st, f, p0 + q0, Hq, Vq);
+    else
+      hipLaunchKernelGGL(dft_final_kernel<2>, grid, dim3(256), smem, st, f, p0 + q0, Hq, Vq);
   }
   RTB_HIP(hipGetLastError());
   return RTB_OK;

@@ -4,6 +4,8 @@ import numpy as np
 import pytest
 
 import rustb_amd as ra
+from oracle import oracle as O
+from rustb_amd.model import synth_model
 
 pytestmark = pytest.mark.gpu
 
@@ -54,3 +56,19 @@ def test_paired_sum_at_tile_edges(dim, n, n_R, nk, lone):
                 if gauge == "atom":
                     X = X + 1j * (t[None, :] - t[:, None]) * H
                 assert np.abs(V[some, p] - X * P).max() <= tol * (np.abs(w).max() + 2 * np.abs(t).max() + 1)
+
+
+@pytest.mark.parametrize("mesh,n", [((1, 1), 2), ((3, 2), 3), ((4, 1, 2), 8), ((5, 2, 3), 9), ((16, 2), 11), ((17, 3), 4)])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-10), ("mixed", 1e-6)])
+def test_mesh_sum_at_tile_edges(mesh, n, precision, tol):
+    """The uniform mesh's last pass (4 k-points per thread, 64 elements), with
+    the velocities one by one (fp64) and as one operator (mixed)."""
+    m = synth_model(2, len(mesh), False, n, 1, 40 + n)
+    o = O.model_from_arrays(m.lat, m.orb, m.spin, m.hamR, m.ham)
+    dirs = np.eye(len(mesh))[:2] + 0.1
+    p = ra.Parameters(kmesh=mesh, direction=dirs, mu=np.array([-0.2, 0.3]), eta=0.05, T=np.array([900.0]),
+                      precision=precision)
+    got = m.hall_conductivity(p).conductivity
+    ref = O.hall_conductivity_direct(o, list(mesh), dirs, np.array([-0.2, 0.3]), 900.0, 0.05)
+    # as the products' tests: an eigenvector's error over the gap, times |v|^2 / eta^2
+    assert np.abs(got - ref).max() <= tol * max(np.abs(ref).max(), 1e-2)
