@@ -52,13 +52,15 @@ def device_sync():
 # count per launch group in rtb_stats.flop): the kernels each one times, the
 # arithmetic they run on and that unit's published peak.
 ROOFLINE_STAGES = {
-    "gemm64": ("zgemm3m_kernel<double, ...>", "FP64 matrix cores", PEAK_FP64),
+    "gemm64": ("col_product_kernel + refine_cols_kernel", "FP64 matrix cores", PEAK_FP64),
     "gemm32": ("zgemm3m_kernel<float, ...>", "FP32 matrix cores", PEAK_FP32),
     "tridiag": ("eigh_tridiag_reg_kernel", "vector ALU", None),
     "backtransform": ("eigh_backtrans_reg_kernel", "vector ALU", None),
 }
-# above 128 orbitals the eigensolver's stages are the two-stage route's kernels
-BAND_KERNELS = {"tridiag": "band_reduce_kernel + band_chase_kernel", "backtransform": "band_backtrans_kernel"}
+# above 128 orbitals the eigensolver's stages are the two-stage route's kernels,
+# the products separate ones
+BAND_KERNELS = {"tridiag": "band_reduce_kernel + band_chase_kernel", "backtransform": "band_backtrans_kernel",
+                "gemm64": "zgemm3m_kernel<double, ...>"}
 
 
 def traffic_from_profiles(stage, workload="wannier3d-n128"):
@@ -308,7 +310,8 @@ def energy_cut_bench(args):
         "stage_ms_per_step": {names[i]: round(st["ms"][i], 2) for i in range(len(names))},
         "sigma_mu0": float(sig[mu.size // 2]),
         "roofline": {"bound": "mfma", "achieved": round(tf, 3), "peak": 78.6, "unit": "TFLOP/s",
-                     "frac": round(tf / 78.6, 4), "traffic": None, "kernel": "zgemm3m_kernel<double, ...>",
+                     "frac": round(tf / 78.6, 4), "traffic": None,
+                     "kernel": "zgemm3m_kernel<double, ...>" if model.nsta > 128 else "col_product_kernel",
                      "stage": "gemm64", "note": "the overlap and Kubo products; host_ms = the walk schedule, launches and synchronisations"},
     }
     if not args.no_cpu and args.ec_workload == "random2d-n32":
