@@ -4,8 +4,9 @@
 // Algorithm (the LAPACK zheevx route for the tridiagonal part):
 //   1. Householder reduction to a real symmetric tridiagonal T = Q^H A Q
 //      (zhetd2 with zlarfg reflectors): tridiag_reg in eigh_reg.hpp;
-//   2. eigenvalues of T by Sturm-count bisection, one thread per eigenvalue
-//      (dstebz's counting rule with the pivmin guard): bisect_all;
+//   2. eigenvalues of T, one thread per eigenvalue: Sturm-count bisection
+//      (dstebz's counting rule with the pivmin guard) and, once a bracket holds
+//      one eigenvalue, Newton steps kept inside it: bisect_all;
 //   3. eigenvectors of T: for an isolated eigenvalue the top-down and
 //      bottom-up factorisations of T - lam I and the twist index (the vector
 //      itself is generated where it is consumed, in backtrans_reg); inside a
@@ -151,22 +152,32 @@ RTB_HD inline void gershgorin(int n, const T* d, const T* e, T& gl, T& gu) {
 // it, log2(n) bisection steps shorter.
 //
 // It bisects until the bracket holds no other eigenvalue, then takes Newton
-// steps on the characteristic polynomial inside the bracket (a step that leaves
-// it bisects); once a step says that the root is within the tolerance, counts
-// on both sides of it are the bracket bisection would have ended with: 7 walks
-// of the recurrence (10 in the slowest thread of 64) instead of 46 in FP64, 17
-// in FP32.
+// steps on the characteristic polynomial inside the bracket; once a step says
+// that the root is within the tolerance, counts on both sides of it are the
+// bracket bisection would have ended with.  A step that leaves the bracket or is
+// not half as long as the one before it bisects: next to m close eigenvalues
+// outside the bracket Newton steps shrink by 1 - 1 / (m + 1) only.  So does any
+// walk that finds the bracket wider than `bound`, 2^8 times its first width w
+// times 0.6 per walk: by induction the bracket stays below w 2^8 0.6^(t - 1) after
+// t walks, whatever the counts are, and the loop ends with a bracket within the
+// tolerance after at most 1 + (8 + log2(w / tol)) / log2(1 / 0.6) walks, 78 in
+// FP64 and 39 in FP32 at n = 32 (76 and 36 at 128).
+// Measured walks per eigenvalue (the slowest of 64): levels that repel each other
+// 8.5 (12) in FP64 and 7 (11) in FP32, bisection alone 47 and 18; flat bands of n/2
+// to n - 3 equal levels with others 1e-8 to 1e-1 beside them, whose equal levels
+// bisect to the end, 34 (47, worst 64) and 15 (20, worst 37).
 // Every bracket end is a point whose count was taken, brackets of neighbours
 // separate at a common point and a value lies in its bracket, so the
-// eigenvalues are ascending and as close as by bisection alone; near-degenerate
-// ones bisect to the end.  Each round is one walk of the same kind in every
+// eigenvalues are ascending and as close as by bisection alone.
+// Each round is one walk of the same kind in every
 // thread (threads in different phases share it; with a walk of its own per
 // phase a wave ran them one after the other: 357 us where bisection took 132).
 // The walk is a serial chain, the walks are the stage's time: FP64 n = 36, 301
 // matrices, 132 -> 56 us; FP32 n = 128, 15798 matrices with the twisted
 // factorisations 1.43 -> 1.11 ms.
+// walks: the walks taken per eigenvalue (for checks on the host), or null.
 template <typename T, typename Team>
-RTB_HD void bisect_all(Team& tm, int n, const T* d, const T* e, T* e2, T* E, T* cnt) {
+RTB_HD void bisect_all(Team& tm, int n, const T* d, const T* e, T* e2, T* E, T* cnt, int* walks = nullptr) {
   for (int i = tm.id; i < n; i += tm.nt) e2[i] = (i + 1 < n) ? e[i] * e[i] : T(0);
   tm.sync();
   T gl, gu;
@@ -216,13 +227,15 @@ RTB_HD void bisect_all(Team& tm, int n, const T* d, const T* e, T* e2, T* E, T* 
     int clo = a > 0 ? static_cast<int>(cnt[a - 1]) : 0, chi = a < n - 1 ? static_cast<int>(cnt[a]) : n;
     T x = T(0.5) * (lo + hi), prev = Lim<T>::huge();
     int check = 0;  // 1, 2: x is the lower, upper end of a predicted bracket
-    for (int it = 0; it < 200; ++it) {
+    T bound = fmin(T(256) * (hi - lo), Lim<T>::huge());
+    int it = 0;
+    for (;; ++it) {
       const T tol = atol + T(2) * eps * fmax(fabs(lo), fabs(hi));
       if (hi - lo <= tol) break;
       if (!(x > lo && x < hi)) {
         check = 0;
         x = T(0.5) * (lo + hi);
-        if (x <= lo || x >= hi) break;
+        if (!(x > lo && x < hi)) break;  // adjacent numbers; NaN or infinite ends
       }
       T dlog;
       const int c = sturm_newton(n, d, e2, x, pivmin, dlog);
@@ -236,7 +249,11 @@ RTB_HD void bisect_all(Team& tm, int n, const T* d, const T* e, T* e2, T* E, T* 
       }
       const T mid = T(0.5) * (lo + hi);
       T next = mid;
-      if (clo == j && chi == j + 1) {
+      bound *= T(0.6);
+      if (!(hi - lo <= bound)) {
+        check = 0;
+        prev = Lim<T>::huge();
+      } else if (clo == j && chi == j + 1) {
         if (check == 1 && below) {
           next = root + T(0.5) * tol;
           check = 2;
@@ -258,7 +275,7 @@ RTB_HD void bisect_all(Team& tm, int n, const T* d, const T* e, T* e2, T* E, T* 
               have = next >= hi;
             }
             prev = as;
-          } else if (xn > lo && xn < hi) {
+          } else if (xn > lo && xn < hi && as < T(0.5) * prev) {
             next = xn;
             prev = as;
           } else {
@@ -270,6 +287,7 @@ RTB_HD void bisect_all(Team& tm, int n, const T* d, const T* e, T* e2, T* E, T* 
       x = next;
     }
     E[j] = have ? root : T(0.5) * (lo + hi);
+    if (walks) walks[j] = it + (have ? 1 : 0);
   }
   tm.sync();
 }

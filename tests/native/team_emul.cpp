@@ -130,7 +130,28 @@ int run_band(int n, const double* H, double* E, double* Z, int vectors, int rows
   return 0;
 }
 
+// One thread for all eigenvalues of a tridiagonal matrix, with the walks each took.
+struct OneThread {
+  int id = 0, nt = 1;
+  void sync() {}
+};
+
+template <typename T>
+void run_tridiag_eigenvalues(int n, const double* d, const double* e, double* E, int* walks) {
+  OneThread tm;
+  std::vector<T> D(d, d + n), Ee(e, e + n), e2(n), Ev(n), cnt(n);
+  rtb::bisect_all<T>(tm, n, D.data(), Ee.data(), e2.data(), Ev.data(), cnt.data(), walks);
+  for (int j = 0; j < n; ++j) E[j] = static_cast<double>(Ev[j]);
+}
+
 }  // namespace
+
+extern "C" void emul_tridiag_eigenvalues(int n, int fp32, const double* d, const double* e, double* E, int* walks) {
+  if (fp32)
+    run_tridiag_eigenvalues<float>(n, d, e, E, walks);
+  else
+    run_tridiag_eigenvalues<double>(n, d, e, E, walks);
+}
 
 extern "C" int emul_eigh_band(int n, int fp32, const double* H, double* E, double* Z, int vectors, int rows_out) {
   if (n < 2 || n > 256) return -1;

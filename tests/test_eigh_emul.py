@@ -13,6 +13,7 @@ import subprocess
 
 import numpy as np
 import pytest
+import scipy.linalg as sl
 import scipy.linalg.lapack as L
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -35,6 +36,16 @@ def emul(tmp_path_factory):
         assert rc == 0
         return E, (Z.T if rows_out else Z)
 
+    def eigenvalues(d, e, fp32):
+        d = np.ascontiguousarray(d)
+        n = d.size
+        e = np.append(e, 0.0)
+        E, walks = np.zeros(n), np.zeros(n, np.int32)
+        p = [a.ctypes.data_as(ctypes.c_void_p) for a in (d, e, E, walks)]
+        lib.emul_tridiag_eigenvalues(n, fp32, *p)
+        return E, walks
+
+    run.eigenvalues = eigenvalues
     return run
 
 
@@ -115,6 +126,68 @@ def test_reg_clustered_spectra(emul, case):
     assert np.abs(E - w).max() < 1e-13
     assert np.abs(H @ Z - Z * E).max() < 1e-13
     assert np.abs(Z.conj().T @ Z - np.eye(n)).max() < 1e-13
+
+
+def flat_bands(n, m, rng):
+    """Spectra of m (nearly) equal levels with a level above them, close to one of
+    the n - 1 points the eigenvalue search splits [-1, 1] at, the rest random."""
+    for i in range(12):
+        point = -1.0 + 2.0 * rng.integers(1, n) / n
+        off = 2.0 / n * 10.0 ** rng.uniform(-4.0, -1.3)
+        spread = (0.0, 1e-9)[i % 2] * rng.uniform(-1.0, 1.0, m)
+        # the point between the two, or both on one side of it
+        flat = point - off * rng.choice([0.1, 0.5, -2.0])
+        yield np.concatenate([flat + spread, [flat + off, -1.0, 1.0][: n - m], rng.uniform(-1.0, 1.0, max(n - m - 3, 0))])
+
+
+@pytest.mark.parametrize("fp32", [0, 1])
+@pytest.mark.parametrize("n", [32, 48, 64, 96, 128, 256])
+def test_levels_beside_flat_bands(emul, n, fp32):
+    """An eigenvalue next to a set of close ones, where Newton steps on the
+    characteristic polynomial crawl: every eigenvalue within the rounding of
+    bisection, within the walks the bracket's bound allows."""
+    rng = np.random.default_rng(n)
+    eps = 2.0**-24 if fp32 else 2.0**-53
+    for m in (n // 2, 3 * n // 4, n - 3):
+        for i, w in enumerate(flat_bands(n, m, rng)):
+            d, e = w, np.zeros(n - 1)
+            if i % 3 == 2:  # rotated to a dense matrix and reduced
+                Q, _ = np.linalg.qr(rng.standard_normal((n, n)))
+                T = sl.hessenberg((Q * w) @ Q.T)
+                d, e = np.diag(T).copy(), np.diag(T, -1).copy()
+            if fp32:
+                d, e = d.astype(np.float32).astype(float), e.astype(np.float32).astype(float)
+            E, walks = emul.eigenvalues(d, e, fp32)
+            off = np.abs(np.concatenate([[0.0], e])) + np.abs(np.append(e, 0.0))
+            norm = np.abs(d).max() + off.max()  # of Gershgorin's interval
+            ref = sl.eigvalsh_tridiagonal(d, e, lapack_driver="stebz")  # bisection
+            # brackets of 3 eps each and counts exact for entries moved by a few eps
+            assert np.abs(E - ref).max() <= 16 * eps * norm
+            assert np.all(np.diff(E) >= 0)
+            # first width 2 norm (1 + small) / n, the tolerance at least eps tnorm
+            tnorm = max(abs((d - off).min()), abs((d + off).max()))
+            assert walks.max() <= 2 + (8 + np.log2(2.1 * tnorm / n / (eps * tnorm))) / np.log2(1 / 0.6)
+
+
+@pytest.mark.parametrize("fp32", [0, 1])
+def test_walks_of_separated_levels(emul, fp32):
+    """Levels that repel each other: about 8 walks each, not a bisection's 47 (18)."""
+    rng = np.random.default_rng(4)
+    A = rng.standard_normal((128, 128))
+    T = sl.hessenberg(A + A.T)
+    _, walks = emul.eigenvalues(np.diag(T).copy(), np.diag(T, -1).copy(), fp32)
+    assert walks.mean() < 10 and walks.max() <= 20
+
+
+@pytest.mark.parametrize("fp32", [0, 1])
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf, 1e308, 0.0, 1e-320])
+def test_eigenvalue_search_ends(emul, fp32, bad):
+    """Entries at and past the number range: the search ends."""
+    d = np.linspace(-1.0, 1.0, 9)
+    for dd, ee in ((np.where(np.arange(9) == 4, bad, d), np.full(8, 0.3)), (d, np.where(np.arange(8) == 3, bad, 0.3)),
+                   (np.full(9, bad), np.full(8, bad))):
+        _, walks = emul.eigenvalues(dd, ee, fp32)
+        assert walks.max() < 2200
 
 
 @pytest.mark.parametrize("n,fp32", [(9, 0), (64, 0), (128, 0), (100, 1)])
