@@ -1048,7 +1048,6 @@ struct BerryBufs {
   int *dperm = nullptr, *dbounds = nullptr;
   double *dlpart = nullptr, *dlsum = nullptr, *dlay = nullptr;
   EigBufs eb{};
-  int total_blk = 0;
 };
 
 static int berry_alloc(Work& w, const rtb_model* m, const BerryJob& j, size_t K, const std::vector<Chunk>& chunks,
@@ -1077,14 +1076,15 @@ static int berry_alloc(Work& w, const rtb_model* m, const BerryJob& j, size_t K,
     b.dZ = b.dH;  // H is consumed by the Householder kernel before Z is written
   }
   if (rterm) RTB_TRY(w.alloc(&b.rproj, static_cast<size_t>(m->nR) * n2 * 2));
-  b.total_blk = 0;
   if (j.mode == 2) {
-    for (const Chunk& ch : chunks) b.total_blk += hall_blocks(ch.c);
+    // one chunk's partial sums: each chunk's are added up before the next
+    int rows = 0;
+    for (const Chunk& ch : chunks) rows = std::max(rows, hall_blocks(ch.c, static_cast<int>(j.n_mu)));
     RTB_TRY(w.alloc(&b.dmu, j.n_mu));
-    RTB_TRY(w.alloc(&b.dpart, static_cast<size_t>(b.total_blk) * j.n_mu));
+    RTB_TRY(w.alloc(&b.dpart, static_cast<size_t>(rows) * j.n_mu));
     RTB_TRY(w.alloc(&b.dsig, j.n_mu));
     if (j.geometry) {
-      RTB_TRY(w.alloc(&b.dmpart, static_cast<size_t>(b.total_blk) * j.n_mu));
+      RTB_TRY(w.alloc(&b.dmpart, static_cast<size_t>(rows) * j.n_mu));
       RTB_TRY(w.alloc(&b.dmsig, j.n_mu));
     }
   }
@@ -1189,7 +1189,6 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
   double *dmu = bb.dmu, *dpart = bb.dpart, *dsig = bb.dsig, *docc = bb.docc, *dmpart = bb.dmpart;
   double* dmsig = bb.dmsig;
   EigBufs& eb = bb.eb;
-  const int total_blk = bb.total_blk;
   double* T1 = bb.kub;
   double* A = bb.kub + K * n2 * 2;
   double* B = bb.kub + K * n2 * 4;
@@ -1202,7 +1201,6 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
   size_t chunk_no = 0;
   std::vector<double> kp;
   std::vector<double> sums(j.mode == 2 ? j.n_mu : 0), msums(j.mode == 2 && j.geometry ? j.n_mu : 0);
-  int blk_off = 0;
   for (const Chunk& ch : chunks) {
     const size_t k0 = ch.k0, c = ch.c;
     if (j.k) {
@@ -1282,14 +1280,14 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
       ++l2;
       RTB_TRY(to_host(st, w, j.occ + k0, docc, c * sizeof(double)));
     } else {
-      const int nb = hall_blocks(c);
-      RTB_TRY(hall_partials(st, n, c, j.dipole ? dKern : dOm, dE, dmu, static_cast<int>(j.n_mu), j.T,
-                            dpart + static_cast<size_t>(blk_off) * j.n_mu, nb, j.dipole));
-      ++l2;
+      const int n_mu = static_cast<int>(j.n_mu), nb = hall_blocks(c, n_mu);
+      RTB_TRY(hall_partials(st, n, c, j.dipole ? dKern : dOm, dE, dmu, n_mu, j.T, dpart, nb, j.dipole));
+      RTB_TRY(reduce_partials(st, dpart, nb, n_mu, 1.0, dsig, chunk_no > 0));
+      l2 += 2;
       if (j.geometry) {
-        RTB_TRY(hall_partials(st, n, c, dMet, dE, dmu, static_cast<int>(j.n_mu), j.T,
-                              dmpart + static_cast<size_t>(blk_off) * j.n_mu, nb));
-        ++l2;
+        RTB_TRY(hall_partials(st, n, c, dMet, dE, dmu, n_mu, j.T, dmpart, nb));
+        RTB_TRY(reduce_partials(st, dmpart, nb, n_mu, 1.0, dmsig, chunk_no > 0));
+        l2 += 2;
       }
       if (j.n_layers > 0) {  // Zc still holds the eigenvector columns
         RTB_TRY(layer_partials(st, n, c, Zc, f32 ? dsc : nullptr, dE, dOm, dmu, static_cast<int>(j.n_mu), j.T,
@@ -1298,7 +1296,6 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
                                 bb.dlsum + chunk_no * ml));
         l2 += 2;
       }
-      blk_off += nb;
     }
     RTB_TRY(tmr.end(l2));
     if (j.mode != 2 && &ch != &chunks.back()) {  // the last chunk's outputs come with the counters
@@ -1308,10 +1305,6 @@ static int berry_run(const rtb_model* m, BerryJob& j, Exec& ex) {
     ++chunk_no;
   }
   if (j.mode == 2) {
-    RTB_TRY(tmr.begin(RTB_STAGE_REDUCE));
-    RTB_TRY(reduce_partials(st, dpart, total_blk, static_cast<int>(j.n_mu), 1.0, dsig));
-    if (j.geometry) RTB_TRY(reduce_partials(st, dmpart, total_blk, static_cast<int>(j.n_mu), 1.0, dmsig));
-    RTB_TRY(tmr.end(j.geometry ? 2 : 1));
     RTB_TRY(to_host(st, w, sums.data(), dsig, j.n_mu * sizeof(double)));
     if (j.geometry) RTB_TRY(to_host(st, w, msums.data(), dmsig, j.n_mu * sizeof(double)));
     if (j.n_layers > 0) {

@@ -253,7 +253,7 @@ int hall_partials(hipStream_t st, int n, size_t nk, const double* omega, const d
 // A[k * sk + n * sb] (om: [nk][n]).
 int dipole_combine(hipStream_t st, int n, size_t nk, const double* A2, const double* A3, size_t sk, size_t sb,
                    const double* om1, const double* om2, bool sym, double* out);
-int hall_blocks(size_t nk);
+int hall_blocks(size_t nk, int n_mu);
 // out[k][m] = sum_n omega[k][n] f(E[k][n], mu_m, T) per k-point ([nk][n_mu]).
 int kterms(hipStream_t st, int n, size_t nk, const double* omega, const double* E, const double* mu, int n_mu,
            double T, double* out);
@@ -303,8 +303,9 @@ int abs2(hipStream_t st, size_t total, const double* z, double* x);
 int dos_partials(hipStream_t st, size_t ne, const double* evals, double Emin, double dE, int En,
                  double sigma, double* partial, int n_blk);
 int dos_blocks(size_t ne, int En);
-// out[j] = scale * sum_blk partial[blk][j]
-int reduce_partials(hipStream_t st, const double* partial, int n_blk, int m, double scale, double* out);
+// out[j] = scale * sum_blk partial[blk][j], added to out[j] with add
+int reduce_partials(hipStream_t st, const double* partial, int n_blk, int m, double scale, double* out,
+                    bool add = false);
 // out[j] = sum over n_rows rows of partial[r][j] (one workgroup per column, a
 // fixed order): for many rows and few columns.
 int column_sums(hipStream_t st, const double* partial, size_t n_rows, int m, double* out);

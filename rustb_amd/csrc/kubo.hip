@@ -139,26 +139,33 @@ __global__ void __launch_bounds__(256) layer_partials_kernel(int n, const double
     partial[k * n_mu * n_layers + o] = (wred[0][o] + wred[1][o]) + (wred[2][o] + wred[3][o]);
 }
 
-// Band sums per block of kHallK k-points and up to kHallMu chemical
-// potentials: the block's kHallK n values of E and omega are read once, in
+// Band sums per block of kper (hall_points) k-points and up to kHallMu chemical
+// potentials: the block's kper n values of E and omega are read once, in
 // order, by consecutive threads, each value weighted for all the mu; the
 // threads' sums are added in a fixed order.  (A thread per k-point walking its
 // n bands once per mu read E and omega n_mu times, strided: n = 32, 131072
 // k-points, 41 mu at 300 K 3.4 ms, now 0.34 ms.)  Bound: the exponentials.
 constexpr int kHallK = 64;
 constexpr int kHallMu = 8;
+// k-points per block: 64, and 256 (a quarter of the partial rows) where those
+// blocks alone come to four per CU (n = 2, 1024 x 1024, 2100 mu: the sums 11.9
+// ms with 64 everywhere, 6.2 ms; n = 8, 256 x 256, 200 mu 0.226, 0.201 ms).
+int hall_points(size_t nk, int n_mu) {
+  const size_t big = (nk + 4 * kHallK - 1) / (4 * kHallK) * static_cast<size_t>((n_mu + kHallMu - 1) / kHallMu);
+  return big >= 1024 ? 4 * kHallK : kHallK;
+}
 
 // deriv: weights -df/dE = f (1 - f) / width (fermi_derivative_from_width,
 // thermodynamics.rs:122-126) instead of f
 __global__ void __launch_bounds__(256) hall_partials_kernel(int n, size_t nk, const double* __restrict__ omega,
                                                             const double* __restrict__ E,
                                                             const double* __restrict__ mu, int n_mu, double width,
-                                                            int deriv, double* __restrict__ partial) {
+                                                            int deriv, int kper, double* __restrict__ partial) {
   __shared__ double red[kHallMu][4];
   const int m0 = blockIdx.y * kHallMu;
   const int nm = n_mu - m0 < kHallMu ? n_mu - m0 : kHallMu;
-  const size_t k0 = blockIdx.x * static_cast<size_t>(kHallK);
-  const size_t cnt = (nk - k0 < static_cast<size_t>(kHallK) ? nk - k0 : static_cast<size_t>(kHallK)) * n;
+  const size_t k0 = blockIdx.x * static_cast<size_t>(kper);
+  const size_t cnt = (nk - k0 < static_cast<size_t>(kper) ? nk - k0 : static_cast<size_t>(kper)) * n;
   const double* __restrict__ Eb = E + k0 * n;
   const double* __restrict__ ob = omega + k0 * n;
   double m[kHallMu], s[kHallMu];
@@ -223,7 +230,7 @@ __global__ void __launch_bounds__(256) segment_sums_kernel(const double* __restr
 // out[j] = sum_r partial[r][j] for r < n_rows: one workgroup per column,
 // strided partial sums then a fixed tree (for many rows).
 __global__ void __launch_bounds__(256) column_sums_kernel(const double* __restrict__ partial, size_t n_rows, int m,
-                                                          double scale, double* __restrict__ out) {
+                                                          double scale, int add, double* __restrict__ out) {
   __shared__ double red[256];
   const int j = blockIdx.x;
   double acc = 0.0;
@@ -234,7 +241,7 @@ __global__ void __launch_bounds__(256) column_sums_kernel(const double* __restri
     if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[j] = red[0] * scale;
+  if (threadIdx.x == 0) out[j] = (add ? out[j] : 0.0) + red[0] * scale;
 }
 
 constexpr int kDosE = 256;   // energies per block
@@ -269,13 +276,13 @@ __global__ void dos_partials_kernel(size_t ne, int chunk, const double* __restri
   partial[static_cast<size_t>(blockIdx.y) * En + j] = acc;
 }
 
-__global__ void reduce_partials_kernel(const double* __restrict__ partial, int n_blk, int m, double scale,
+__global__ void reduce_partials_kernel(const double* __restrict__ partial, int n_blk, int m, double scale, int add,
                                        double* __restrict__ out) {
   const int j = blockIdx.x * 256 + threadIdx.x;
   if (j >= m) return;
   double s = 0.0;
   for (int b = 0; b < n_blk; ++b) s += partial[static_cast<size_t>(b) * m + j];
-  out[j] = s * scale;
+  out[j] = (add ? out[j] : 0.0) + s * scale;
 }
 
 // Omega_n = sum_{m != n} -2 Im(A_nm B_mn) / ((E_n - E_m)^2 + eta^2) from A
@@ -470,7 +477,10 @@ int abs2(hipStream_t st, size_t total, const double* z, double* x) {
   return RTB_OK;
 }
 
-int hall_blocks(size_t nk) { return static_cast<int>((nk + kHallK - 1) / kHallK); }
+int hall_blocks(size_t nk, int n_mu) {
+  const int kper = hall_points(nk, n_mu);
+  return static_cast<int>((nk + kper - 1) / kper);
+}
 
 int hall_partials(hipStream_t st, int n, size_t nk, const double* omega, const double* E, const double* mu,
                   int n_mu, double T, double* partial, int n_blk, bool deriv) {
@@ -478,7 +488,7 @@ int hall_partials(hipStream_t st, int n, size_t nk, const double* omega, const d
   hipLaunchKernelGGL(hall_partials_kernel,
                      dim3(static_cast<unsigned>(n_blk), static_cast<unsigned>((n_mu + kHallMu - 1) / kHallMu)),
                      dim3(256), 0, st, n, nk, omega, E, mu, n_mu, T <= 0.0 ? 0.0 : T * 8.617333262145e-5,
-                     deriv ? 1 : 0, partial);
+                     deriv ? 1 : 0, hall_points(nk, n_mu), partial);
   RTB_HIP(hipGetLastError());
   return RTB_OK;
 }
@@ -504,7 +514,8 @@ int segment_sums(hipStream_t st, const double* term, const long long* start, int
 
 int column_sums(hipStream_t st, const double* partial, size_t n_rows, int m, double* out) {
   if (m == 0) return RTB_OK;
-  hipLaunchKernelGGL(column_sums_kernel, dim3(static_cast<unsigned>(m)), dim3(256), 0, st, partial, n_rows, m, 1.0, out);
+  hipLaunchKernelGGL(column_sums_kernel, dim3(static_cast<unsigned>(m)), dim3(256), 0, st, partial, n_rows, m, 1.0, 0,
+                     out);
   RTB_HIP(hipGetLastError());
   return RTB_OK;
 }
@@ -529,16 +540,16 @@ int dos_partials(hipStream_t st, size_t ne, const double* evals, double Emin, do
 // A thread per column walks the rows one after the other (1024 rows x 41: 0.32
 // ms); from this many rows on a workgroup per column (a fixed tree: 0.01 ms).
 constexpr int kReduceRows = 32;
-int reduce_partials(hipStream_t st, const double* partial, int n_blk, int m, double scale, double* out) {
+int reduce_partials(hipStream_t st, const double* partial, int n_blk, int m, double scale, double* out, bool add) {
   if (m == 0) return RTB_OK;
   if (n_blk >= kReduceRows) {
     hipLaunchKernelGGL(column_sums_kernel, dim3(static_cast<unsigned>(m)), dim3(256), 0, st, partial,
-                       static_cast<size_t>(n_blk), m, scale, out);
+                       static_cast<size_t>(n_blk), m, scale, add ? 1 : 0, out);
     RTB_HIP(hipGetLastError());
     return RTB_OK;
   }
   hipLaunchKernelGGL(reduce_partials_kernel, dim3(static_cast<unsigned>((m + 255) / 256)), dim3(256), 0, st,
-                     partial, n_blk, m, scale, out);
+                     partial, n_blk, m, scale, add ? 1 : 0, out);
   RTB_HIP(hipGetLastError());
   return RTB_OK;
 }

@@ -65,6 +65,25 @@ def test_hall_sums_at_block_edges(mesh, n_mu, T):
     assert np.abs(got - ref).max() <= 1e-10 * max(np.abs(ref).max(), 1e-3)
 
 
+@pytest.mark.parametrize("mesh,n_mu", [((90, 91), 9), ((300, 220), 41), ((171, 181), 70)])
+def test_hall_sums_over_chunks(mesh, n_mu, monkeypatch):
+    """The occupation sums in blocks of 64 and of 256 k-points, in one chunk
+    and added up over several, for the curvature, the metric and the dipole."""
+    m = synth_model(3, 2, False, 3, 1, 17, n_R_target=9)
+    p = ra.Parameters(kmesh=mesh, direction=np.eye(2), mu=np.linspace(-1.0, 1.3, n_mu), eta=0.05, T=np.array([300.0]))
+    d = ra.Parameters(kmesh=mesh, direction=np.array([[1.0, 0.0], [0.0, 1.0], [1.0, 1.0]]), mu=p.mu, eta=0.05, T=p.T)
+
+    def call():
+        g = m.quantum_geometry(p)
+        return [m.hall_conductivity(p).conductivity, g.metric, g.berry_curvature, m.extrinsic_nonlinear_hall(d).conductivity]
+
+    one = call()
+    monkeypatch.setenv("RTB_WORKSPACE_MB", "6")
+    for a, b in zip(one, call()):
+        # sums of nk terms in another order
+        assert np.abs(a - b).max() <= 1e-11 * max(np.abs(a).max(), 1e-3)
+
+
 @pytest.mark.parametrize("mesh,En", [((1, 1), 1), ((5, 7), 256), ((33, 31), 257), ((200, 90), 801)])
 def test_dos_at_block_edges(mesh, En):
     """The DOS in blocks of 64 to 2048 eigenvalues and 256 energies."""

@@ -46,6 +46,19 @@ def test_noalloc_matches_hall_direct_twice(prec):
         assert np.abs(out - ref).max() <= tol * max(np.abs(ref).max(), 1e-3), (mesh, out, ref)
 
 
+def test_noalloc_large_mesh_many_chemical_potentials():
+    """1024 x 1024 k-points and 2100 chemical potentials: the partial sums of
+    one chunk at a time fit the scratch beside the chunk's matrices."""
+    lib = _lib.load()
+    model, _ = random_pair(2, False, 2, 2, seed=44)
+    mu, dirs = np.linspace(-2.0, 2.0, 2100), np.eye(2)
+    rc, ref = hall(lib.rtb_hall_direct, model, (1024, 1024), mu, dirs, 0, T=100.0)
+    assert rc == 0
+    rc, out = hall(lib.rtb_hall_direct_noalloc, model, (1024, 1024), mu, dirs, 0, T=100.0)
+    assert rc == 0, lib.rtb_last_error()
+    assert np.abs(out - ref).max() <= 1e-10 * np.abs(ref).max()
+
+
 def test_noalloc_rejects_what_does_not_fit():
     lib = _lib.load()
     model, _ = random_pair(2, False, 2, 2, seed=43)
