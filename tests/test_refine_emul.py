@@ -8,6 +8,7 @@ import subprocess
 
 import numpy as np
 import pytest
+import scipy.linalg as sl
 import scipy.linalg.lapack as L
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -28,6 +29,14 @@ def rr(tmp_path_factory):
                             E.ctypes.data_as(ctypes.c_void_p), ctypes.c_double(gap_rel))
         return Z, E
 
+    def small(G, M):
+        c = G.shape[0]
+        G, M = np.ascontiguousarray(G), np.ascontiguousarray(M)
+        ev, X = np.zeros(c), np.zeros((c, c), np.complex128)
+        sweeps = lib.emul_cluster_small(c, *[a.ctypes.data_as(ctypes.c_void_p) for a in (G, M, ev, X)])
+        return sweeps, ev, X
+
+    run.small = small
     return run
 
 
@@ -88,3 +97,29 @@ def test_no_cluster_is_identity(rr):
     H, Z, HZ, E = fp32_like_pairs(rng, n, eig)
     Zr, Er = rr(Z.copy(), HZ, E.copy(), 1e-3)
     assert np.array_equal(Er, E) and np.array_equal(Zr, Z)
+
+
+@pytest.mark.parametrize("spread", [0.0, 1e-17, 1e-16, 1e-15, 1e-13, 1e-10, 1e-6])
+@pytest.mark.parametrize("level", [-0.3, 0.0, 7.0])
+def test_small_problem_ends_at_equal_levels(rr, spread, level):
+    """The c x c problem of equal levels, their spread from nothing past the
+    rounding of the level: values and vectors to rounding, in the sweeps a
+    quadratic iteration takes."""
+    rng = np.random.default_rng(8)
+
+    def herm(c):
+        A = rng.standard_normal((c, c)) + 1j * rng.standard_normal((c, c))
+        return 0.5 * (A + A.conj().T)
+
+    for c in (2, 3, 5, 8):
+        for _ in range(20):
+            G = np.eye(c) + 1e-13 * herm(c)
+            M = level * G + spread * herm(c)
+            sweeps, ev, X = rr.small(G, M)
+            assert 0 <= sweeps <= 8
+            # entries of order |level| + c spread, c^2 operations on each
+            tol = 4 * c * c * np.finfo(float).eps
+            ref = sl.eigvalsh(M - level * G, G) + level
+            assert np.abs(ev - ref).max() <= tol * (abs(level) + c * spread)
+            assert np.abs(X.conj().T @ G @ X - np.eye(c)).max() <= tol
+            assert np.abs(X.conj().T @ M @ X - np.diag(ev)).max() <= tol * (abs(level) + c * spread)
