@@ -204,7 +204,10 @@ __global__ void __launch_bounds__(256) cut_kernel(cut::View V, const double* __r
 // energy, to LDS and then take the item's sub-simplices of every chemical
 // potential, one per lane (1, 3 or 1 of a tetrahedron with one, two or three
 // vertices below mu, 1 or 2 of a triangle), each lane running the whole band
-// sums of its quadrature points from broadcast LDS reads.  The sub-simplices
+// sums of its quadrature points from broadcast LDS reads; up to 32 sub-simplices
+// share the wave's lanes evenly, 2 to 32 for each one's band sum, added in a fixed
+// butterfly (n = 32, 128 x 128, 256 mu over the band width: the call 12.2 ms with
+// one lane each, 6.0 ms).  The sub-simplices
 // of a mu are added in a fixed order, items follow each other in a fixed order
 // within a wave, a wave's sums are per mu, and the full items enter as steps
 // (one value at their first full mu, summed up at the end), so the result
@@ -357,7 +360,12 @@ __global__ void __launch_bounds__(256) cut_mu_kernel(cut::View V, const double* 
       const int i2 = DIM == 3 ? first(i1, a1, e[DIM - 1] + cut::kEps, true) : a1;
       const int n1 = i1 - a0, n2 = i2 - i1;
       const int units = n1 + DIM * n2 + (a1 - i2);
-      for (int u = lane; u < units; u += 64) {
+      // few units: `parts` lanes (a power of two) split each one's band sum
+      int sh = 0;
+      while (sh < 5 && units << (sh + 1) <= 64) ++sh;
+      const int parts = 1 << sh;
+      for (int q = lane; q < units << sh; q += 64) {
+        const int u = q >> sh;
         int i, kind;
         if (u < n1) {
           i = a0 + u;
@@ -414,37 +422,47 @@ __global__ void __launch_bounds__(256) cut_mu_kernel(cut::View V, const double* 
 #pragma unroll
             for (int d = 0; d < NV; ++d) en[k] = fma(sE[y.b * NV + d], lam[k][d], en[k]);
           }
-          for (int mb = 0; mb < n; ++mb) {
-            if (mb == y.b) continue;  // the same in every lane
-            double ev[NV], kv[NV];
-#pragma unroll
-            for (int d = 0; d < NV; ++d) {
-              ev[d] = sE[mb * NV + d];
-              kv[d] = sK[mb * NV + d];
-            }
-#pragma unroll
-            for (int k = 0; k < NV; ++k) {
-              double de = en[k], kk = 0.0;
+          const auto terms = [&](int first_mb, int step_mb) {
+            for (int mb = first_mb; mb < n; mb += step_mb) {
+              if (mb == y.b) continue;
+              double ev[NV], kv[NV];
 #pragma unroll
               for (int d = 0; d < NV; ++d) {
-                de = fma(-ev[d], lam[k][d], de);
-                kk = fma(kv[d], lam[k][d], kk);
+                ev[d] = sE[mb * NV + d];
+                kv[d] = sK[mb * NV + d];
               }
-              const double denom = fma(de, de, eta2);
-              // hardware reciprocal and two Newton steps; a division where
-              // those would leave the number range
-              double r = __builtin_amdgcn_rcp(denom);
-              r = fma(r, fma(-denom, r, 1.0), r);
-              r = fma(r, fma(-denom, r, 1.0), r);
-              if (!(denom < 1e300)) r = 1.0 / denom;
-              if (!(denom < 1e-30)) im[k] = fma(kk, r, im[k]);
+#pragma unroll
+              for (int k = 0; k < NV; ++k) {
+                double de = en[k], kk = 0.0;
+#pragma unroll
+                for (int d = 0; d < NV; ++d) {
+                  de = fma(-ev[d], lam[k][d], de);
+                  kk = fma(kv[d], lam[k][d], kk);
+                }
+                const double denom = fma(de, de, eta2);
+                // hardware reciprocal and two Newton steps; a division where
+                // those would leave the number range
+                double r = __builtin_amdgcn_rcp(denom);
+                r = fma(r, fma(-denom, r, 1.0), r);
+                r = fma(r, fma(-denom, r, 1.0), r);
+                if (!(denom < 1e300)) r = 1.0 / denom;
+                if (!(denom < 1e-30)) im[k] = fma(kk, r, im[k]);
+              }
             }
-          }
+          };
+          if (sh == 0)
+            terms(0, 1);  // one band at a time in the whole wave
+          else
+            terms(q & (parts - 1), parts);
+          // the lanes of a unit hold the same vol and take the same branch
+          for (int o = parts / 2; o > 0; o >>= 1)
+#pragma unroll
+            for (int k = 0; k < NV; ++k) im[k] += __shfl_xor(im[k], o);
           constexpr double wq = 1.0 / NV;
 #pragma unroll
           for (int k = 0; k < NV; ++k) val += vol * wq * (-2.0 * im[k]);
         }
-        sub[u] = kind == 4 ? -val : val;
+        if ((q & (parts - 1)) == 0) sub[u] = kind == 4 ? -val : val;
       }
       tm.wave_sync();
       // the sub-simplices of each mu, in order
@@ -811,22 +829,23 @@ static size_t energy_cut_waves(int dim, size_t nx, size_t ny, size_t nz, int n) 
   return (total + 255) / 256 * 4;
 }
 
-// Lanes over mu (cut_mu_kernel) from a full wave of chemical potentials on, if
-// there are at least 3/2 of them per mesh division: a band's spread over a cell
-// is about its width over the divisions, so below that an item is cut once or
-// not at all and most lanes idle.  Whole calls, mu over the band width, split
-// band sum against lanes over mu: n = 32 on 128 x 128, 64 mu 10.6 / 11.9 ms,
-// 128 mu 12.4 / 12.9, 256 mu 15.6 / 13.3; n = 96 on 24 x 24, 64 mu 11.8 / 8.3;
-// n = 12 on 20 x 18 x 16, 64 mu 6.7 / 2.2, 512 mu 48 / 3.5.
-static bool lanes_over_mu(size_t nx, size_t ny, size_t nz, size_t n_mu) {
-  return n_mu >= 64 && 2 * n_mu >= 3 * std::max(nx, std::max(ny, nz));
-}
+// Lanes over mu (cut_mu_kernel) from 64 chemical potentials on.  Whole calls, split
+// band sum against lanes over mu, for windows of 0.05, 1 and 30 band widths, in ms:
+//   2D n = 32, 128 x 128    64 mu  5.36/4.72  4.87/4.97  4.54/4.47
+//                          256 mu  8.36/5.18  6.39/6.01  5.19/4.69
+//   2D n = 4, 200 x 200     64 mu  3.38/3.16  3.23/3.29  3.10/3.11
+//   2D n = 96, 24 x 24      64 mu  10.6/5.82  6.74/5.26  4.39/4.38
+//   3D n = 12, 20 x 18 x 16 64 mu  9.57/1.49  4.65/1.86  1.13/1.09
+// With fewer the split band sum is up to 5% ahead where an item is cut once or not at
+// all (n = 12, 20 x 18 x 16, 4 mu 1.40/1.11  1.07/1.12  0.89/0.91), the lanes over mu in
+// narrow windows only.
+static bool lanes_over_mu(size_t n_mu) { return n_mu >= 64; }
 // partial rows (waves); with lanes over mu a wave covers one or more groups of
 // 64 items, so that the rows stay few
 constexpr size_t kCutMuRows = 8192;
 size_t energy_cut_rows(int dim, size_t nx, size_t ny, size_t nz, int n, size_t n_mu) {
   const size_t waves = energy_cut_waves(dim, nx, ny, nz, n);
-  return lanes_over_mu(nx, ny, nz, n_mu) ? std::min(waves, kCutMuRows) : waves;
+  return lanes_over_mu(n_mu) ? std::min(waves, kCutMuRows) : waves;
 }
 
 namespace {
@@ -865,7 +884,7 @@ int energy_cut_t0(hipStream_t st, int dim, size_t nx, size_t ny, size_t nz, int 
   const size_t waves = energy_cut_waves(dim, nx, ny, nz, n);
   const unsigned blocks = static_cast<unsigned>(waves / 4);
   const cut::View V{n, E, Ki, 1, perm};
-  if (lanes_over_mu(nx, ny, nz, n_mu)) {
+  if (lanes_over_mu(n_mu)) {
     const size_t rows = energy_cut_rows(dim, nx, ny, nz, n, n_mu);
     const size_t smem = 4 * cut_mu_wave_doubles(n, dim + 1) * sizeof(double);
     for (size_t m0 = 0; m0 < n_mu; m0 += chunk) {

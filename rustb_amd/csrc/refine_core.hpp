@@ -105,7 +105,7 @@ RTB_RHD inline bool cluster_rr_small(int c, C2 (*buf)[kMaxCluster][kMaxCluster],
   // is the cluster's mean level: the rotations then round relative to the spread
   // within the cluster.  Without it equal levels never met the bound below, each
   // rotation rounding at eps |level|, and all 30 sweeps ran (25 on average at a
-  // spread of 1e-17, now 1); 4000 k-points with 24 equal levels of 32: the kernel
+  // spread of 1e-17, now 2); 4000 k-points with 24 equal levels of 32: the kernel
   // that calls this 53 ms, now 12 ms.
   double shift = 0.0;
   for (int a = 0; a < c; ++a) shift += P[a][a].re;

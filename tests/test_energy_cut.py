@@ -709,3 +709,27 @@ def test_gpu_many_chemical_potentials_equal_few(dim, n, mesh, n_mu):
                           for i in range(0, n_mu, 40)])
     assert np.abs(ref).max() > 0 or 1 in mesh
     np.testing.assert_allclose(got, ref, rtol=0, atol=1e-11 * max(np.abs(ref).max(), 1e-3))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window", [0.02, 1.0, 20.0])
+@pytest.mark.parametrize("dim,n,mesh", [(2, 1, (9, 8)), (2, 3, (31, 30)), (2, 31, (12, 11)), (2, 33, (25, 2)),
+                                        (3, 2, (6, 5, 7)), (3, 33, (3, 4, 3))])
+def test_gpu_chemical_potentials_per_item(dim, n, mesh, window):
+    """64 chemical potentials over windows in which a simplex is cut at none, a few
+    or all of them (2 to 32 lanes, or one, per cut) against 40 and 24 of them."""
+    from rustb_amd.model import synth_model
+
+    m = synth_model(1 if dim == 3 else 3, dim, False, n, 1, 190 + n, scale=0.5, decay=1.0,
+                    n_R_target=0 if dim == 3 else 9)
+    e = m.solve_band_all(np.zeros((1, dim)))[0, n // 2]
+    mu = e + window * 1.5 * math.sqrt(n) * np.linspace(-1.0, 1.0, 64)
+    d = np.eye(dim)[:2]
+
+    def call(x):
+        p = ra.Parameters(kmesh=mesh, direction=d, mu=x, eta=0.02, integration="EnergyCut")
+        return m.hall_conductivity(p).conductivity
+
+    got, ref = call(mu), np.concatenate([call(mu[:40]), call(mu[40:])])
+    # two orders of the same FP64 sums, n * cells terms
+    np.testing.assert_allclose(got, ref, rtol=0, atol=1e-11 * max(np.abs(ref).max(), 1e-3))
