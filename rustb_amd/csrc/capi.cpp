@@ -1730,9 +1730,11 @@ int rtb_hall_energy_cut(const rtb_model* m, const size_t* kmesh, const double* m
   RTB_TRY(tmr.end(1));
   const double width = T <= 0.0 ? 0.0 : T * 8.617333262145e-5;  // thermodynamics.rs:10, 50-59
   RTB_TRY(energy_cut_convolve(mu, n_mu, width, [&](const double* mv, size_t nm, double* s0) -> int {
-    // partial rows of at most 512 MB (at least one column)
+    // partial rows of at most 512 MB (at least one column), and at most 2^20
+    // columns: a launch holds fewer than 2^32 threads, 65536 rows of workgroups
     const size_t rows = energy_cut_rows(m->dim, nx, ny, nz, n, nm);
-    const size_t chunk = std::max<size_t>(1, std::min<size_t>(nm, (size_t(512) << 20) / (rows * sizeof(double))));
+    const size_t chunk = std::max<size_t>(
+        1, std::min({nm, size_t(1) << 20, (size_t(512) << 20) / (rows * sizeof(double))}));
     double *dmu, *ds0, *dpart;
     RTB_TRY(w.alloc(&dmu, nm));
     RTB_TRY(w.alloc(&ds0, nm));

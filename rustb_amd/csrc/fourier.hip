@@ -214,7 +214,8 @@ __global__ void __launch_bounds__(kBlock, NP == 3 && KT == 2 ? 2 : 3) fourier_de
 template <int NP, int KT>
 int launch_tiles(hipStream_t st, const FourierArgs& a, const double* k, size_t nk, double* H, double* V) {
   const size_t n2 = static_cast<size_t>(a.n) * a.n, etiles = (n2 + kPairElems - 1) / kPairElems;
-  const size_t maxk = (size_t(1) << 30) / etiles / (16 * KT) * (16 * KT);  // tiles of a launch within an int
+  // a launch holds fewer than 2^32 threads: at most 2^23 tiles
+  const size_t maxk = (size_t(1) << 23) / etiles * (16 * KT);
   const size_t vk = NP == 2 && a.combine ? 1 : NP;
   for (size_t off = 0; off < nk; off += maxk) {
     const size_t cnt = std::min(nk - off, maxk), ktiles = (cnt + 16 * KT - 1) / (16 * KT);

@@ -539,10 +539,13 @@ int dos_partials(hipStream_t st, size_t ne, const double* evals, double Emin, do
 
 // A thread per column walks the rows one after the other (1024 rows x 41: 0.32
 // ms); from this many rows on a workgroup per column (a fixed tree: 0.01 ms).
+// A launch holds fewer than 2^32 threads (beyond, the grid is cut short without an
+// error), so more than 2^23 columns stay with a thread each.
 constexpr int kReduceRows = 32;
+constexpr int kReduceCols = 1 << 23;
 int reduce_partials(hipStream_t st, const double* partial, int n_blk, int m, double scale, double* out, bool add) {
   if (m == 0) return RTB_OK;
-  if (n_blk >= kReduceRows) {
+  if (n_blk >= kReduceRows && m <= kReduceCols) {
     hipLaunchKernelGGL(column_sums_kernel, dim3(static_cast<unsigned>(m)), dim3(256), 0, st, partial,
                        static_cast<size_t>(n_blk), m, scale, add ? 1 : 0, out);
     RTB_HIP(hipGetLastError());

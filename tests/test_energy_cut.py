@@ -733,3 +733,20 @@ def test_gpu_chemical_potentials_per_item(dim, n, mesh, window):
     got, ref = call(mu), np.concatenate([call(mu[:40]), call(mu[40:])])
     # two orders of the same FP64 sums, n * cells terms
     np.testing.assert_allclose(got, ref, rtol=0, atol=1e-11 * max(np.abs(ref).max(), 1e-3))
+
+
+@pytest.mark.gpu
+def test_gpu_more_chemical_potentials_than_a_launch_holds():
+    """2^24 + 1 chemical potentials on a 2 x 2 mesh against every 2^18-th of them."""
+    from rustb_amd.model import synth_model
+
+    m = synth_model(3, 2, False, 3, 1, 5, scale=0.5, decay=1.0, n_R_target=9)
+    mu = np.linspace(-1.0, 1.0, 2**24 + 1)
+
+    def call(x):
+        p = ra.Parameters(kmesh=(2, 2), direction=np.eye(2), mu=x, eta=0.02, integration="EnergyCut")
+        return m.hall_conductivity(p).conductivity
+
+    ref = call(mu[:: 2**18])
+    assert np.abs(ref[-8:]).min() > 1e-3 * np.abs(ref).max()
+    np.testing.assert_allclose(call(mu)[:: 2**18], ref, rtol=0, atol=1e-12 * np.abs(ref).max())

@@ -93,3 +93,14 @@ def test_dos_at_block_edges(mesh, En):
     Er, rr = O.dos(o, list(mesh), -4.0, 4.0, En, 0.05)
     # sums of nk positive terms in another order: nk eps of the result
     assert np.abs(rho - rr).max() <= 1e-11 * max(np.abs(rr).max(), 1e-300)
+
+
+def test_dos_with_more_energies_than_workgroups_of_a_launch():
+    """2^24 + 1 energies over 32 blocks of eigenvalues: a workgroup per energy
+    would be 2^32 threads, more than a launch holds."""
+    m = ra.workloads.graphene()
+    E, rho = m.dos((128, 256), -4.0, 4.0, 2**24 + 1, 0.05)
+    Er, rr = m.dos((128, 256), -4.0, 4.0, 2**8 + 1, 0.05)
+    np.testing.assert_allclose(E[:: 2**16], Er, rtol=0, atol=1e-14)
+    # the same terms in another order: nk eps, and the energies' rounding over sigma
+    np.testing.assert_allclose(rho[:: 2**16], rr, rtol=0, atol=1e-11 * rr.max())
