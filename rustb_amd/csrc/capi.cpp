@@ -187,10 +187,13 @@ size_t workspace_budget() {
   return std::min(it->second / 8, size_t(32) << 30);
 }
 
+// At most 2^25 k-points: a launch holds fewer than 2^32 threads (beyond, the grid is
+// cut short without an error), and the small matrices that many would fit of take
+// 64 threads each.
 size_t chunk_for(size_t nk, size_t per_k_bytes) {
   const size_t budget = workspace_budget();
   size_t c = std::max<size_t>(1, budget / std::max<size_t>(per_k_bytes, 1));
-  return std::min(nk, c);
+  return std::min({nk, c, size_t(1) << 25});
 }
 
 // Bytes per k-point of alloc_eig's buffers beyond those of n <= 128 (the

@@ -104,3 +104,14 @@ def test_dos_with_more_energies_than_workgroups_of_a_launch():
     np.testing.assert_allclose(E[:: 2**16], Er, rtol=0, atol=1e-14)
     # the same terms in another order: nk eps, and the energies' rounding over sigma
     np.testing.assert_allclose(rho[:: 2**16], rr, rtol=0, atol=1e-11 * rr.max())
+
+
+def test_more_k_points_than_a_launch_holds(monkeypatch):
+    """8200 x 8200 k-points of one band fit the workspace at once, but at a
+    workgroup of 64 threads each they are more than 2^32 threads."""
+    m = synth_model(3, 2, False, 1, 1, 5, n_R_target=9)
+    one = m.dos((8200, 8200), -2.0, 2.0, 11, 0.3)[1]
+    monkeypatch.setenv("RTB_WORKSPACE_MB", "2000")
+    many = m.dos((8200, 8200), -2.0, 2.0, 11, 0.3)[1]
+    # sums of nk positive terms in another order
+    np.testing.assert_allclose(one, many, rtol=1e-11)
