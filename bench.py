@@ -52,7 +52,7 @@ def device_sync():
 # count per launch group in rtb_stats.flop): the kernels each one times, the
 # arithmetic they run on and that unit's published peak.
 ROOFLINE_STAGES = {
-    "gemm64": ("col_product_kernel + refine_cols_kernel", "FP64 matrix cores", PEAK_FP64),
+    "gemm64": ("col_product_kernel + refine_cols_kernel", "FP64 (and FP32) matrix cores", PEAK_FP64),
     "gemm32": ("zgemm3m_kernel<float, ...>", "FP32 matrix cores", PEAK_FP32),
     "tridiag": ("eigh_tridiag_reg_kernel", "vector ALU", None),
     "backtransform": ("eigh_backtrans_reg_kernel", "vector ALU", None),
@@ -426,8 +426,18 @@ def main():
     f32 = args.precision == "mixed" and dname in ("tridiag", "backtransform")
     if peak is None:  # vector ALU: FP32 in the mixed form, FP64 otherwise
         peak = PEAK_FP32 if f32 else PEAK_FP64
-    per_launch_ms = stage_ms[dom] / stage_launch[dom]
-    flop_per_launch = stage_flop[dom] / stage_launch[dom]
+    # up to 128 orbitals the FP64 products' stage is two kernels per chunk, which
+    # form several of the products rtb_stats counts; in the mixed form the FP32
+    # correction products are in one of them, so in that stage's time
+    fused = n <= 128 and dname == "gemm64"
+    g32 = names.index("gemm32")
+    launches = 2.0 * stage_launch[names.index("tridiag")] if fused else stage_launch[dom]
+    mflop32 = stage_mflop[g32] if fused else 0.0
+    per_launch_ms = stage_ms[dom] / launches
+    flop32 = stage_flop[g32] if fused else 0.0
+    flop_per_launch = (stage_flop[dom] + flop32) / launches
+    if flop32 > 0:  # of the stage's mix
+        peak = round((stage_flop[dom] + flop32) / (stage_flop[dom] / PEAK_FP64 + flop32 / PEAK_FP32), 2)
     achieved = flop_per_launch / (per_launch_ms * 1e-3) / 1e12
     roofline = {
         "bound": "mfma",
@@ -440,7 +450,7 @@ def main():
         "stage": dname,
         "arithmetic": unit_name,
         "per_launch_ms": round(per_launch_ms, 4),
-        "launches_per_step": int(round(stage_launch[dom] / args.steps)),
+        "launches_per_step": int(round(launches / args.steps)),
         "algorithmic_flop_per_launch": flop_per_launch,
         "dominant_stage_by_time": names[int(np.argmax(stage_ms[:ns - 1]))],
     }
@@ -448,12 +458,15 @@ def main():
         # what the matrix cores executed (3M products, padded tiles) against
         # the rate this device attains on independent MFMA chains
         ceil = mfma_ceiling()
-        executed = stage_mflop[dom] / stage_launch[dom] / (per_launch_ms * 1e-3) / 1e12
+        executed = (stage_mflop[dom] + mflop32) / (stage_ms[dom] * 1e-3) / 1e12
         roofline["mfma_executed"] = round(executed, 3)
         if ceil:
+            # the time of the executed operations at the chains' rates: the peak is
+            # that of the stage's mix of FP64 and FP32
             att = ceil["fp64_mfma" if dname == "gemm64" else "fp32_mfma"]
-            roofline["attainable_peak"] = att
-            roofline["frac_of_attainable"] = round(executed / att, 4)
+            t_att = stage_mflop[dom] / att + mflop32 / ceil["fp32_mfma"]
+            roofline["attainable_peak"] = round((stage_mflop[dom] + mflop32) / t_att, 2)
+            roofline["frac_of_attainable"] = round(t_att / 1e12 / (stage_ms[dom] * 1e-3), 4)
     out = {
         "metric": METRIC,
         "value": round(value, 2),
